@@ -14,6 +14,13 @@
 //      buffer once.
 // Blocks are persistent (grid = resident capacity) and loop over element
 // blocks, so the reference matrices are staged once per block.
+//
+// The Global operator (GLOBAL kernels, StageArgs::global) is the same
+// semi-discrete operator with fully upwinded SMA faces and conductivity, so it
+// runs here and no matrix is read: 24 Np values per element and stage instead
+// of the matrix's 190 entries per row at order 3 (10,368 tetrahedra with no two
+// alike, FP32 order 3: 659 us per stage from the assembled matrix, 13.2 us
+// here).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -27,20 +34,20 @@ namespace {
 
 using namespace valu;
 
-template <int P, typename T, int MODE>
+template <int P, typename T, int MODE, bool GLOBAL>
 __global__ __launch_bounds__(256) void dg_stage_kernel(StageArgs<T> a)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     stage_load_ref<P, T>(a.mats, a.tabs, smem_raw);
     __syncthreads();
-    for (int blk = blockIdx.x; blk < a.nblk; blk += gridDim.x) stage_block<P, T, MODE>(a, smem_raw, blk);
+    for (int blk = blockIdx.x; blk < a.nblk; blk += gridDim.x) stage_block<P, T, MODE, GLOBAL>(a, smem_raw, blk);
 }
 
 template <int P, typename T, int MODE>
 hipError_t launch_one(const StageArgs<T>& a, int grid, hipStream_t s)
 {
     constexpr size_t bytes = Smem<P, T>::bytes;
-    auto kern = dg_stage_kernel<P, T, MODE>;
+    auto kern = a.global ? dg_stage_kernel<P, T, MODE, true> : dg_stage_kernel<P, T, MODE, false>;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(256), bytes, s, a);
     return hipGetLastError();
 }
@@ -62,8 +69,9 @@ hipError_t launch_mode(const StageArgs<T>& a, int mode, int grid, hipStream_t s)
 template <int P, typename T, int MODE>
 void set_smem_attr()
 {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(dg_stage_kernel<P, T, MODE>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)Smem<P, T>::bytes);
+    for (const void* kern : {reinterpret_cast<const void*>(dg_stage_kernel<P, T, MODE, false>),
+                             reinterpret_cast<const void*>(dg_stage_kernel<P, T, MODE, true>)})
+        (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Smem<P, T>::bytes);
 }
 
 // Raises the dynamic-LDS limit of every stage variant of this order (needed
@@ -79,7 +87,7 @@ int occupancy_one()
     set_smem_attr<P, T, kModeRk2>();
     set_smem_attr<P, T, kModeRk3>();
     set_smem_attr<P, T, kModeRk4>();
-    auto kern = dg_stage_kernel<P, T, kModeLserk>;
+    auto kern = dg_stage_kernel<P, T, kModeLserk, false>;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, 256, bytes) != hipSuccess) return 1;
     return nb > 0 ? nb : 1;
 }

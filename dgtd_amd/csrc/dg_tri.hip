@@ -43,7 +43,9 @@ struct TSmem {
     static constexpr size_t bytes = sizeof(T) * (size_t)nReal + sizeof(int) * (size_t)nInt;
 };
 
-template <int P, typename T, int MODE>
+// GLOBAL: the Global operator's form (fully upwinded SMA edges, conductivity;
+// see stage_body.hpp).
+template <int P, typename T, int MODE, bool GLOBAL>
 __global__ __launch_bounds__(256) void dg_tri_stage(StageArgs<T> a)
 {
     using S = TShape<P>;
@@ -139,12 +141,15 @@ __global__ __launch_bounds__(256) void dg_tri_stage(StageArgs<T> a)
             const int nb = sC[el * kTriConn + f];
             const T* uM = uMs[k];
             T* d = ds[k];
+            T alpha = a.alpha;
             if (nb >= 0) {
 #pragma unroll
                 for (int c = 0; c < 6; ++c) d[c] -= uM[c];
             } else {
+                if constexpr (GLOBAL)
+                    if (-nb - 1 == 3 || -nb - 1 == 6) alpha = T(1);
                 T ce, ch;
-                bc_coeffs<T>(-nb - 1, a.alpha, ce, ch);
+                bc_coeffs<T>(-nb - 1, alpha, ce, ch);
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
                     d[c] = ce * uM[c];
@@ -155,12 +160,12 @@ __global__ __launch_bounds__(256) void dg_tri_stage(StageArgs<T> a)
             const T ndE = nx * d[0] + ny * d[1];
             const T ndH = nx * d[3] + ny * d[4];
             // n = (nx, ny, 0):  fH_x = -n_y dE_z + n_z dE_y + a (dH_x - ndH n_x), ...
-            const T fHx = -ny * d[2] + a.alpha * (d[3] - ndH * nx);
-            const T fHy = nx * d[2] + a.alpha * (d[4] - ndH * ny);
-            const T fHz = -nx * d[1] + ny * d[0] + a.alpha * d[5];
-            const T fEx = ny * d[5] + a.alpha * (d[0] - ndE * nx);
-            const T fEy = -nx * d[5] + a.alpha * (d[1] - ndE * ny);
-            const T fEz = nx * d[4] - ny * d[3] + a.alpha * d[2];
+            const T fHx = -ny * d[2] + alpha * (d[3] - ndH * nx);
+            const T fHy = nx * d[2] + alpha * (d[4] - ndH * ny);
+            const T fHz = -nx * d[1] + ny * d[0] + alpha * d[5];
+            const T fEx = ny * d[5] + alpha * (d[0] - ndE * nx);
+            const T fEy = -nx * d[5] + alpha * (d[1] - ndE * ny);
+            const T fEz = nx * d[4] - ny * d[3] + alpha * d[2];
             T* o = sF + el * NF + m;
             o[0 * EB * NF] = fEx * fs;
             o[1 * EB * NF] = fEy * fs;
@@ -186,6 +191,9 @@ __global__ __launch_bounds__(256) void dg_tri_stage(StageArgs<T> a)
                     rv[c] = a.res[c * N + idx];
                 if constexpr (MODE == kModeRk2 || MODE == kModeRk3) xv[c] = a.x[c * N + idx];
             }
+            T sg = T(0);
+            if constexpr (GLOBAL)
+                if (a.sig != nullptr) sg = a.sig[e0 + el];
             T ar[6], as[6], lf[6];
 #pragma unroll
             for (int c = 0; c < 6; ++c) { ar[c] = T(0); as[c] = T(0); lf[c] = T(0); }
@@ -214,6 +222,10 @@ __global__ __launch_bounds__(256) void dg_tri_stage(StageArgs<T> a)
             rhs[3] = (-Dy(2) + lf[3]) * g[14];         // H_x: -dEz/dy
             rhs[4] = (Dx(2) + lf[4]) * g[14];          // H_y:  dEz/dx
             rhs[5] = (-Dx(1) + Dy(0) + lf[5]) * g[14]; // H_z: -(dEy/dx - dEx/dy)
+            if constexpr (GLOBAL) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) rhs[c] -= sg * sQ[c * EB * NP + el * NP + i];
+            }
 #pragma unroll
             for (int c = 0; c < 6; ++c) {
                 const size_t o = c * N + idx;
@@ -247,7 +259,7 @@ template <int P, typename T, int MODE>
 hipError_t tri_launch_one(const StageArgs<T>& a, int grid, hipStream_t s)
 {
     constexpr size_t bytes = TSmem<P, T>::bytes;
-    auto kern = dg_tri_stage<P, T, MODE>;
+    auto kern = a.global ? dg_tri_stage<P, T, MODE, true> : dg_tri_stage<P, T, MODE, false>;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(256), bytes, s, a);
     return hipGetLastError();
 }
@@ -255,8 +267,9 @@ hipError_t tri_launch_one(const StageArgs<T>& a, int grid, hipStream_t s)
 template <int P, typename T, int MODE>
 void tri_set_attr()
 {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(dg_tri_stage<P, T, MODE>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)TSmem<P, T>::bytes);
+    for (const void* kern : {reinterpret_cast<const void*>(dg_tri_stage<P, T, MODE, false>),
+                             reinterpret_cast<const void*>(dg_tri_stage<P, T, MODE, true>)})
+        (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)TSmem<P, T>::bytes);
 }
 
 template <int P, typename T>

@@ -150,7 +150,10 @@ struct dgtd_op {
     int grid_cfg[dgtd::kMfmaConfigs] = {};        // grid per configuration, 0 = does not fit
     // autotuning record: candidates timed at creation (or taken from the cache)
     dgtd_tuning tuning{};
-    // assembled operator (DGTD_KERNEL_CSR)
+    // Global operator (DGTD_KERNEL_CSR): matrix-free on tetrahedra and
+    // triangles (sigma/eps_r per element, NULL = no conductivity), else assembled
+    bool global_free = false;
+    void* d_sig = nullptr;
     int64_t* d_rowptr = nullptr;
     uint16_t* d_col = nullptr;
     int* d_etab = nullptr;
@@ -207,7 +210,7 @@ struct dgtd_op {
         for (void* p : {d_geo, (void*)d_conn, d_mats, d_mats_mfma, (void*)d_order, (void*)d_tabs, (void*)d_M, (void*)d_jac,
                         (void*)d_eps, (void*)d_mu, (void*)d_partials, (void*)d_out3, (void*)d_unstable, (void*)d_probe_elem,
                         (void*)d_tfsf_elem, (void*)d_tfsf_sign, (void*)d_tfsf_xyz, (void*)d_tfsf_geo,
-                        (void*)d_lift, (void*)d_waves, (void*)d_rowptr, (void*)d_col, (void*)d_etab, d_val,
+                        (void*)d_lift, (void*)d_waves, d_sig, (void*)d_rowptr, (void*)d_col, (void*)d_etab, d_val,
                         (void*)d_probe_w, (void*)d_probe_out, d_buf[0],
                         d_buf[1], d_buf[2], d_buf[3]})
             if (p) (void)hipFree(p);
@@ -235,13 +238,15 @@ struct dgtd_op {
         a.val = static_cast<const T*>(d_val);
         a.nrows = ndofs;
         a.nnz = nnz;
+        a.global = global_free;
+        a.sig = static_cast<const T*>(d_sig);
         return a;
     }
 
     template <typename T>
     hipError_t launch_on(const dgtd::StageArgs<T>& a0, int mode, int var, hipStream_t s) const
     {
-        if (var == DGTD_KERNEL_CSR) return dgtd::launch_csr_stage<T>(a0, mode, s);
+        if (var == DGTD_KERNEL_CSR && !global_free) return dgtd::launch_csr_stage<T>(a0, mode, s);
         if (hex) return dgtd::launch_hex_stage<T>(H3.p, a0, mode, s);
         if (var == DGTD_KERNEL_MFMA) {
             dgtd::StageArgs<T> a = a0;
@@ -616,6 +621,21 @@ void upload_csr(dgtd_op* op, const dgtd::Csr& A)
     op->d_val = op->precision == 64 ? upload(A.val) : upload(dgtd::cast_vec<float>(A.val));
 }
 
+// The Global operator on tetrahedra and triangles: their per-node stage
+// applies it without a matrix (StageArgs::global).  What the assembly refuses
+// is refused here too, so an operator exists for exactly the meshes whose
+// matrix dgtd_global_assemble returns.
+void setup_global(dgtd_op* op, const double* sigma, const std::vector<double>& eps)
+{
+    dgtd::check_global(op->Np, op->K, sigma);
+    if (sigma) {
+        std::vector<double> sg(op->K);
+        for (int e = 0; e < op->K; ++e) sg[e] = sigma[e] / eps[e];
+        op->d_sig = op->precision == 64 ? upload(sg) : upload(dgtd::cast_vec<float>(sg));
+    }
+    op->global_free = true;
+}
+
 // Persistent grid of the matrix-core stage: enough blocks for the tasks, at
 // most the resident ones, in whole XCD groups (the kernel splits the tasks
 // per XCD).
@@ -740,7 +760,7 @@ void create_tri(dgtd_op* op, const dgtd_mesh_desc* mesh, int kernel)
     }
     if (kernel == DGTD_KERNEL_MFMA && op->grid_cfg[0] <= 0)
         throw std::runtime_error("the MFMA kernel does not fit this order and precision, or a state buffer reaches 4 GiB");
-    select_variant(op, kernel, [&] { upload_csr(op, dgtd::assemble_global_tri(md, R, mesh->sigma, op->alpha)); });
+    select_variant(op, kernel, [&] { setup_global(op, mesh->sigma, md.eps); });
 }
 
 // Set-up of a quadrilateral-mesh operator (dim = 2, nvert = 4): the
@@ -1132,8 +1152,7 @@ int dgtd_op_create(const dgtd_mesh_desc* mesh, const dgtd_opts* opts, dgtd_op** 
         if (any_mfma) op->d_order = static_cast<int*>(upload(morton_task_order(mesh)));
         if (opts->kernel == DGTD_KERNEL_MFMA && op->grid_cfg[0] <= 0)
             throw std::runtime_error("the MFMA kernel does not fit this order and precision, or a state buffer reaches 4 GiB");
-        select_variant(op, opts->kernel,
-                       [&] { upload_csr(op, dgtd::assemble_global_tet(md, op->R, mesh->sigma, op->alpha)); });
+        select_variant(op, opts->kernel, [&] { setup_global(op, mesh->sigma, md.eps); });
     } catch (const HipError& e) {
         delete op;
         return fail(DGTD_E_HIP, e.what());
@@ -1689,7 +1708,7 @@ int dgtd_op_work_per_element(const dgtd_op* op, double* bytes, double* flops)
     if (!op) return fail(DGTD_E_ARG, "NULL argument");
     const double s = (double)op->real_size();
     const double Np = op->Np, Nfp = op->Nfp;
-    if (op->variant == DGTD_KERNEL_CSR) {
+    if (op->variant == DGTD_KERNEL_CSR && !op->global_free) {
         // per entry its value and 16-bit column code; per row its pointer,
         // its share of the block's element table (32 ints per 16 rows) and
         // the LSERK vectors (state, residual in/out, out)

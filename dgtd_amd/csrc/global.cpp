@@ -33,6 +33,15 @@
 
 namespace dgtd {
 
+void check_global(int Np, int K, const double* sigma)
+{
+    if (6.0 * Np * (double)K > 2147483647.0) throw std::runtime_error("mesh too large for 32-bit column indices");
+    if (sigma)  // Material.cpp:14 refuses negative conductivity
+        for (int e = 0; e < K; ++e)
+            if (!(sigma[e] >= 0.0) || !std::isfinite(sigma[e]))
+                throw std::runtime_error("conductivity must be finite and >= 0");
+}
+
 namespace {
 
 // BC weights of the own trace (same table as the device kernels).
@@ -242,10 +251,7 @@ void element_block(const ElemView& v, double alpha, double sigma, BlockAcc& acc)
 template <typename View>
 void assemble(int K, int Np, int nf, View&& view_of, const double* sigma, double alpha, Csr& out)
 {
-    if (sigma)  // Material.cpp:14 refuses negative conductivity
-        for (int e = 0; e < K; ++e)
-            if (!(sigma[e] >= 0.0) || !std::isfinite(sigma[e]))
-                throw std::runtime_error("conductivity must be finite and >= 0");
+    check_global(Np, K, sigma);
     const size_t N = (size_t)Np * K;
     std::vector<int64_t> count(6 * N + 1, 0);
     const int hw = (int)std::max(1u, std::thread::hardware_concurrency());
@@ -328,7 +334,6 @@ CsrLocal16 csr_local16(const Csr& A, int64_t N, int Np)
 
 Csr assemble_global_tet(const MeshData& md, const RefTet& R, const double* sigma, double alpha)
 {
-    if (6.0 * R.Np * (double)md.K > 2147483647.0) throw std::runtime_error("mesh too large for 32-bit column indices");
     Csr out;
     auto view = [&](int e) {
         ElemView v{};
@@ -351,7 +356,6 @@ Csr assemble_global_tet(const MeshData& md, const RefTet& R, const double* sigma
 
 Csr assemble_global_tri(const TriMeshData& md, const RefTri& R, const double* sigma, double alpha)
 {
-    if (6.0 * R.Np * (double)md.K > 2147483647.0) throw std::runtime_error("mesh too large for 32-bit column indices");
     Csr out;
     auto view = [&](int e) {
         ElemView v{};
@@ -378,7 +382,6 @@ namespace dgtd {
 
 Csr assemble_global_quad(const TriMeshData& md, const RefQuad& R, const double* sigma, double alpha)
 {
-    if (6.0 * R.Np * (double)md.K > 2147483647.0) throw std::runtime_error("mesh too large for 32-bit column indices");
     Csr out;
     auto view = [&](int e) {
         ElemView v{};
@@ -405,7 +408,6 @@ namespace dgtd {
 
 Csr assemble_global_hex(const HexMeshData& md, const RefHex& R, const double* sigma, double alpha)
 {
-    if (6.0 * R.Np * (double)md.K > 2147483647.0) throw std::runtime_error("mesh too large for 32-bit column indices");
     Csr out;
     auto view = [&](int e) {
         ElemView v{};

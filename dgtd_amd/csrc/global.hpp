@@ -19,6 +19,10 @@ struct Csr {
     std::vector<double> val;
 };
 
+// Throws where the Global operator refuses a mesh of K elements with Np nodes:
+// 32-bit column indices, negative or non-finite conductivity.
+void check_global(int Np, int K, const double* sigma);
+
 // sigma: bulk conductivity per element (NULL = 0).  TF/SF faces are ordinary
 // interior faces here: their injection is a separate, state-independent term.
 Csr assemble_global_tet(const MeshData& md, const RefTet& R, const double* sigma, double alpha);

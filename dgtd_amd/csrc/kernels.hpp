@@ -45,6 +45,11 @@ struct StageArgs {
     int64_t nrows, nnz;
     int np;  // nodes per element
     int* unstable;  // non-null: set to 1 when a stored state entry is unstable (unstable_entry)
+    // matrix-free Global operator on tetrahedra and triangles: the kernels'
+    // Global variant (SMA faces, codes 3 and 6, upwinded fully whatever alpha;
+    // conductivity) with sigma/eps_r per element in sig (NULL = none)
+    bool global;
+    const T* sig;
 };
 
 // Stability test of the reference's time loop (Solver::run, Solver.cpp:499-516,

@@ -56,7 +56,10 @@ __device__ __forceinline__ void stage_load_ref(const T* __restrict__ mats, const
 // One element block (EB elements from e0 = blk*EB) of one stage: gather,
 // flux, curl, LIFT and the stage update.  Starts and ends with a block-wide
 // barrier; the reference matrices must already be in LDS.
-template <int P, typename T, int MODE>
+// GLOBAL: the Global operator's form of the same stage (GlobalEvolution.cpp:
+// 628-1088): SMA faces weighted as at alpha = 1 (DGOperatorFactory.h:485-495,
+// 587-591) and -sigma/eps E on the E rows (:1351-1361).
+template <int P, typename T, int MODE, bool GLOBAL = false>
 __device__ __forceinline__ void stage_block(const StageArgs<T>& a, unsigned char* smem_raw, int blk)
 {
     using S = Shape<P>;
@@ -148,12 +151,15 @@ __device__ __forceinline__ void stage_block(const StageArgs<T>& a, unsigned char
             const T* g = sG + el * kGeoStrideDev;
             const int nb = sC[el * kConnStrideDev + f];
             T* dk = d[k];
+            T alpha = a.alpha;
             if (nb >= 0) {
 #pragma unroll
                 for (int c = 0; c < 6; ++c) dk[c] -= uM[k][c];
             } else {
+                if constexpr (GLOBAL)
+                    if (-nb - 1 == 3 || -nb - 1 == 6) alpha = T(1);
                 T ce, ch;
-                bc_coeffs<T>(-nb - 1, a.alpha, ce, ch);
+                bc_coeffs<T>(-nb - 1, alpha, ce, ch);
 #pragma unroll
                 for (int c = 0; c < 3; ++c) { dk[c] = ce * uM[k][c]; dk[3 + c] = ch * uM[k][3 + c]; }
             }
@@ -164,8 +170,8 @@ __device__ __forceinline__ void stage_block(const StageArgs<T>& a, unsigned char
 #pragma unroll
             for (int x = 0; x < 3; ++x) {
                 const int y = (x + 1) % 3, z = (x + 2) % 3;
-                const T fH = -n3[y] * dk[z] + n3[z] * dk[y] + a.alpha * (dk[3 + x] - ndH * n3[x]);
-                const T fE = n3[y] * dk[3 + z] - n3[z] * dk[3 + y] + a.alpha * (dk[x] - ndE * n3[x]);
+                const T fH = -n3[y] * dk[z] + n3[z] * dk[y] + alpha * (dk[3 + x] - ndH * n3[x]);
+                const T fE = n3[y] * dk[3 + z] - n3[z] * dk[3 + y] + alpha * (dk[x] - ndE * n3[x]);
                 sF[(3 + x) * EB * NF + el * NF + m] = fH * fs;
                 sF[x * EB * NF + el * NF + m] = fE * fs;
             }
@@ -188,6 +194,9 @@ __device__ __forceinline__ void stage_block(const StageArgs<T>& a, unsigned char
                     rv[c] = __builtin_nontemporal_load(a.res + c * N + idx);
                 if constexpr (MODE == kModeRk2 || MODE == kModeRk3) xv[c] = a.x[c * N + idx];
             }
+            T sg = T(0);
+            if constexpr (GLOBAL)
+                if (a.sig != nullptr) sg = a.sig[e0 + el];
             T ar[6], as[6], at[6], lf[6];
 #pragma unroll
             for (int c = 0; c < 6; ++c) { ar[c] = T(0); as[c] = T(0); at[c] = T(0); lf[c] = T(0); }
@@ -217,6 +226,7 @@ __device__ __forceinline__ void stage_block(const StageArgs<T>& a, unsigned char
                 const int y = (x + 1) % 3, z = (x + 2) % 3;
                 rhs[3 + x] = (-Dd(y, z) + Dd(z, y) + lf[3 + x]) * g[26];
                 rhs[x] = (Dd(y, 3 + z) - Dd(z, 3 + y) + lf[x]) * g[25];
+                if constexpr (GLOBAL) rhs[x] -= sg * sQ[x * EB * NP + el * NP + i];
             }
 #pragma unroll
             for (int c = 0; c < 6; ++c) {

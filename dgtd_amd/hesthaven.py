@@ -493,10 +493,12 @@ class HesthavenEvolution:
 
 class GlobalEvolution(HesthavenEvolution):
     """The reference's Global operator (maxwell::GlobalEvolution,
-    src/evolution/GlobalEvolution.cpp:628-1088) on the GPU: the operator
-    assembled into one CSR matrix, applied by a fused SpMV + stage-update
-    kernel, with per-element bulk conductivity sigma (normalised as sigma_SI
-    * Z0, Material.h:30) adding -sigma/eps_r E (DGOperatorFactory.h:1351-1361)."""
+    src/evolution/GlobalEvolution.cpp:628-1088) on the GPU (kernel "csr"), with
+    per-element bulk conductivity sigma (normalised as sigma_SI * Z0,
+    Material.h:30) adding -sigma/eps_r E (DGOperatorFactory.h:1351-1361).
+    Tetrahedra and triangles apply it without a matrix, quadrilaterals and
+    hexahedra as one assembled CSR matrix (a fused SpMV + stage-update
+    kernel); global_assemble returns the matrix of any mesh."""
 
     def __init__(self, vx, EToV, face_bc, order, alpha=1.0, eps=None, mu=None, sigma=None, precision=64,
                  integrator="lserk4", device=0, quads=None):

@@ -129,14 +129,16 @@ typedef struct {
 #define DGTD_KERNEL_VALU 1 /* per-node vector FMA, reference matrices in LDS; on hexahedra the
                             * matrix-free tensor-product stage with the Global operator's flux */
 #define DGTD_KERNEL_MFMA 2 /* matrix cores (v_mfma 16x16x4), 8-element wave tasks */
-/* The assembled operator: the reference's Global operator path
- * (GlobalEvolution::Mult, GlobalEvolution.cpp:628-1088, a CSR SpMV over the
- * matrix DGOperatorFactory::buildGlobalOperator assembles,
- * DGOperatorFactory.h:1428-1600).  The matrix holds the same semi-discrete
- * operator as the matrix-free variants, except that SMA boundary faces weight
- * their upwind terms by 1 whatever alpha, as the Global operator does
+/* The reference's Global operator (GlobalEvolution::Mult,
+ * GlobalEvolution.cpp:628-1088, a CSR SpMV over the matrix
+ * DGOperatorFactory::buildGlobalOperator assembles,
+ * DGOperatorFactory.h:1428-1600; dgtd_global_assemble returns it).  It is the
+ * same semi-discrete operator as the matrix-free variants, except that SMA
+ * faces weight their upwind terms by 1 whatever alpha
  * (DGOperatorFactory.h:485-495, 521-531, 557-567; identical at alpha = 1),
- * plus bulk conductivity; one fused kernel does SpMV and stage update.
+ * plus bulk conductivity.  On tetrahedra and triangles it is applied without
+ * the matrix, by their per-node stage; on quadrilaterals and hexahedra one
+ * fused kernel does the SpMV over the assembled matrix and the stage update.
  * Chosen explicitly (never by autotune) on tetrahedra, triangles and
  * hexahedra (whose AUTO takes their matrix-free stage, DGTD_KERNEL_VALU);
  * the only kernel of quadrilaterals (AUTO selects it there). */
