@@ -343,7 +343,7 @@ def bench_global(D, args, shape="tet"):
         for prec in (32, 64):
             op = D.HesthavenEvolution(vx, E, fbc, order, eps=eps, sigma=sigma, precision=prec,
                                       integrator="lserk4", kernel="valu")
-            st, out[f"matrix_free_fp{prec}"] = timed(op, prec, "hex_stage")
+            st, out[f"matrix_free_fp{prec}"] = timed(op, prec, "tensor_stage")
             out[f"matrix_free_fp{prec}"]["rel_l2_vs_csr"] = float(np.linalg.norm(st - states[prec])
                                                                    / np.linalg.norm(states[prec]))
     out["rel_l2_fp32_vs_fp64"] = float(np.linalg.norm(states[32] - states[64]) / np.linalg.norm(states[64]))

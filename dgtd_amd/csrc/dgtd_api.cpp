@@ -20,7 +20,7 @@
 #include "fields.hpp"
 #include "kernels.hpp"
 #include "trace.hpp"
-#include "hex_dev.hpp"
+#include "tensor_dev.hpp"
 #include "tfsf_host.hpp"
 #include "mesh.hpp"
 #include "packing.hpp"
@@ -247,7 +247,8 @@ struct dgtd_op {
     hipError_t launch_on(const dgtd::StageArgs<T>& a0, int mode, int var, hipStream_t s) const
     {
         if (var == DGTD_KERNEL_CSR && !global_free) return dgtd::launch_csr_stage<T>(a0, mode, s);
-        if (hex) return dgtd::launch_hex_stage<T>(H3.p, a0, mode, s);
+        if (hex) return dgtd::launch_tensor_stage<T>(H3.p, 3, a0, mode, s);
+        if (quad) return dgtd::launch_tensor_stage<T>(Q2.p, 2, a0, mode, s);
         if (var == DGTD_KERNEL_MFMA) {
             dgtd::StageArgs<T> a = a0;
             a.mats = static_cast<const T*>(d_mats_mfma);
@@ -763,8 +764,42 @@ void create_tri(dgtd_op* op, const dgtd_mesh_desc* mesh, int kernel)
     select_variant(op, kernel, [&] { setup_global(op, mesh->sigma, md.eps); });
 }
 
-// Set-up of a quadrilateral-mesh operator (dim = 2, nvert = 4): the
-// assembled operator only.
+// Device records and tables of the matrix-free tensor-product stage: the
+// element records with sigma/eps_r appended, D1 and the two used columns of
+// M1^-1, face nodes and neighbour-node table.
+void upload_tensor(dgtd_op* op, int p, const std::vector<double>& host_geo, const std::vector<int32_t>& conn,
+                   const double* sigma, const std::vector<double>& eps, const std::vector<int>& fmask,
+                   const std::vector<int>& perm)
+{
+    const int K = op->K, n1 = p + 1, stride = (int)(host_geo.size() / K);
+    std::vector<double> geo((size_t)(stride + 1) * K);
+    for (int e = 0; e < K; ++e) {
+        std::copy_n(host_geo.begin() + (size_t)stride * e, stride, geo.begin() + (size_t)(stride + 1) * e);
+        const double sg = sigma ? sigma[e] : 0.0;
+        if (!(sg >= 0.0) || !std::isfinite(sg)) throw std::runtime_error("conductivity must be finite and >= 0");
+        geo[(size_t)(stride + 1) * e + stride] = sg * (1.0 / eps[e]);
+    }
+    const dgtd::Gll1D g1 = dgtd::build_gll1d(p);
+    std::vector<double> m(g1.D.begin(), g1.D.end());
+    for (int i = 0; i < n1; ++i) {
+        m.push_back(g1.Minv[(size_t)i * n1 + 0]);
+        m.push_back(g1.Minv[(size_t)i * n1 + p]);
+    }
+    std::vector<int> tabs(fmask.begin(), fmask.end());
+    tabs.insert(tabs.end(), perm.begin(), perm.end());
+    op->d_tabs = static_cast<int*>(upload(tabs));
+    op->d_conn = static_cast<int*>(upload(conn));
+    if (op->precision == 64) {
+        op->d_geo = upload(geo);
+        op->d_mats = upload(m);
+    } else {
+        op->d_geo = upload(dgtd::cast_vec<float>(geo));
+        op->d_mats = upload(dgtd::cast_vec<float>(m));
+    }
+}
+
+// Set-up of a quadrilateral-mesh operator (dim = 2, nvert = 4): the Global
+// operator only, matrix-free.
 void create_quad(dgtd_op* op, const dgtd_mesh_desc* mesh, int kernel)
 {
     if (kernel != DGTD_KERNEL_CSR && kernel != DGTD_KERNEL_AUTO)
@@ -813,8 +848,12 @@ void create_quad(dgtd_op* op, const dgtd_mesh_desc* mesh, int kernel)
         op->d_tfsf_geo = static_cast<double*>(upload(r.geo));
         op->d_lift = static_cast<double*>(upload(R.LIFT));
     }
+    dgtd::check_global(op->Np, op->K, mesh->sigma);
+    upload_tensor(op, R.p, md.geo, md.conn, mesh->sigma, md.eps, R.Fmask, R.edge_perm);
+    op->global_free = true;
+    op->variant = DGTD_KERNEL_CSR;
+    op->tuning.variant = DGTD_KERNEL_CSR;
     hip_check(hipStreamSynchronize(op->stream), "sync");
-    select_variant(op, DGTD_KERNEL_CSR, [&] { upload_csr(op, dgtd::assemble_global_quad(md, R, mesh->sigma, op->alpha)); });
 }
 
 // Solver::estimateTimeStep (Solver.cpp:302-353).  On tetrahedra under
@@ -912,7 +951,7 @@ dgtd::MeshInput mesh_input(const dgtd_mesh_desc* mesh)
 // operator only.
 // Hexahedra run the Global operator's flux, either assembled (DGTD_KERNEL_CSR)
 // or matrix-free (DGTD_KERNEL_VALU, which DGTD_KERNEL_AUTO selects:
-// hex_stage.hip reads no matrix, and the set-up assembles none).
+// tensor_stage.hip reads no matrix, and the set-up assembles none).
 void create_hex(dgtd_op* op, const dgtd_mesh_desc* mesh, int kernel)
 {
     if (kernel != DGTD_KERNEL_CSR && kernel != DGTD_KERNEL_AUTO && kernel != DGTD_KERNEL_VALU)
@@ -963,48 +1002,7 @@ void create_hex(dgtd_op* op, const dgtd_mesh_desc* mesh, int kernel)
         op->d_lift = static_cast<double*>(upload(R.LIFT));
     }
     if (kernel != DGTD_KERNEL_CSR) {
-        // matrix-free records: geometry with sigma/eps, connectivity, D1 and
-        // the two used columns of M1^-1, face tables
-        const int K = mesh->K, n1 = R.p + 1, Np = R.Np, Nfp = R.Nfp;
-        std::vector<double> geo((size_t)dgtd::kHexGeoDev * K);
-        for (int e = 0; e < K; ++e) {
-            for (int v = 0; v < dgtd::kHexGeoStride; ++v)
-                geo[(size_t)dgtd::kHexGeoDev * e + v] = md.geo[(size_t)dgtd::kHexGeoStride * e + v];
-            const double sg = mesh->sigma ? mesh->sigma[e] : 0.0;
-            if (!(sg >= 0.0) || !std::isfinite(sg)) throw std::runtime_error("conductivity must be finite and >= 0");
-            geo[(size_t)dgtd::kHexGeoDev * e + 35] = sg * md.geo[(size_t)dgtd::kHexGeoStride * e + 33];
-        }
-        const dgtd::Gll1D g1 = dgtd::build_gll1d(R.p);
-        std::vector<double> m(g1.D.begin(), g1.D.end());
-        for (int i = 0; i < n1; ++i) {
-            m.push_back(g1.Minv[(size_t)i * n1 + 0]);
-            m.push_back(g1.Minv[(size_t)i * n1 + R.p]);
-        }
-        std::vector<int> tabs(R.Fmask.begin(), R.Fmask.end());
-        tabs.insert(tabs.end(), R.face_perm.begin(), R.face_perm.end());
-        std::vector<int> fq((size_t)6 * Np, -1);
-        for (int f = 0; f < 6; ++f) {
-            const int axis = f == 0 || f == 5 ? 2 : f == 1 || f == 3 ? 1 : 0;
-            const int stride = axis == 0 ? 1 : axis == 1 ? n1 : n1 * n1;
-            const int b = f == 2 || f == 3 || f == 5 ? R.p : 0;
-            for (int q = 0; q < Nfp; ++q) {
-                const int c = R.Fmask[(size_t)f * Nfp + q];
-                if ((c / stride) % n1 != b) throw std::logic_error("hexahedron face table");
-                for (int i = 0; i < n1; ++i) fq[(size_t)f * Np + c + (i - b) * stride] = q;
-            }
-        }
-        for (int v : fq)
-            if (v < 0) throw std::logic_error("hexahedron normal-line table");
-        tabs.insert(tabs.end(), fq.begin(), fq.end());
-        op->d_tabs = static_cast<int*>(upload(tabs));
-        op->d_conn = static_cast<int*>(upload(md.conn));
-        if (op->precision == 64) {
-            op->d_geo = upload(geo);
-            op->d_mats = upload(m);
-        } else {
-            op->d_geo = upload(dgtd::cast_vec<float>(geo));
-            op->d_mats = upload(dgtd::cast_vec<float>(m));
-        }
+        upload_tensor(op, R.p, md.geo, md.conn, mesh->sigma, md.eps, R.Fmask, R.face_perm);
         hip_check(hipStreamSynchronize(op->stream), "sync");
         op->variant = DGTD_KERNEL_VALU;
         op->tuning.variant = DGTD_KERNEL_VALU;
@@ -1721,6 +1719,12 @@ int dgtd_op_work_per_element(const dgtd_op* op, double* bytes, double* flops)
         const double n1 = op->H3.p + 1.0;
         if (bytes) *bytes = 24.0 * Np * s + 36.0 * s + 48.0;
         if (flops) *flops = Np * (36.0 * n1 + 198.0) + 240.0 * Nfp;
+        return DGTD_OK;
+    }
+    if (op->quad) {  // matrix-free quadrilaterals: state vectors, 19-value record, 8 connectivity ints
+        const double n1 = op->Q2.p + 1.0;
+        if (bytes) *bytes = 24.0 * Np * s + 19.0 * s + 32.0;
+        if (flops) *flops = Np * (24.0 * n1 + 150.0) + 160.0 * Nfp;
         return DGTD_OK;
     }
     if (op->dim == 2) {  // triangles: 2 derivative directions, 3 edges, 15-value record

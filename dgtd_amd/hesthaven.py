@@ -496,7 +496,7 @@ class GlobalEvolution(HesthavenEvolution):
     src/evolution/GlobalEvolution.cpp:628-1088) on the GPU (kernel "csr"), with
     per-element bulk conductivity sigma (normalised as sigma_SI * Z0,
     Material.h:30) adding -sigma/eps_r E (DGOperatorFactory.h:1351-1361).
-    Tetrahedra and triangles apply it without a matrix, quadrilaterals and
+    Tetrahedra, triangles and quadrilaterals apply it without a matrix,
     hexahedra as one assembled CSR matrix (a fused SpMV + stage-update
     kernel); global_assemble returns the matrix of any mesh."""
 

@@ -109,7 +109,8 @@ typedef struct {
                              * Both run the Global operator's flux, the reference's default
                              * operator on its quadrilateral and hexahedral cases
                              * (ExtensiveCasesTest.cpp:1003,1082, Solver3DTest.cpp:57-215):
-                             * quadrilaterals assembled (DGTD_KERNEL_CSR; AUTO selects it),
+                             * quadrilaterals matrix-free under the name DGTD_KERNEL_CSR
+                             * (AUTO selects it),
                              * hexahedra assembled (DGTD_KERNEL_CSR) or matrix-free
                              * (DGTD_KERNEL_VALU, which AUTO selects; sigma allowed). */
 } dgtd_mesh_desc;
@@ -136,9 +137,9 @@ typedef struct {
  * same semi-discrete operator as the matrix-free variants, except that SMA
  * faces weight their upwind terms by 1 whatever alpha
  * (DGOperatorFactory.h:485-495, 521-531, 557-567; identical at alpha = 1),
- * plus bulk conductivity.  On tetrahedra and triangles it is applied without
- * the matrix, by their per-node stage; on quadrilaterals and hexahedra one
- * fused kernel does the SpMV over the assembled matrix and the stage update.
+ * plus bulk conductivity.  On tetrahedra, triangles and quadrilaterals it is
+ * applied without the matrix; on hexahedra one fused kernel does the SpMV over
+ * the assembled matrix and the stage update.
  * Chosen explicitly (never by autotune) on tetrahedra, triangles and
  * hexahedra (whose AUTO takes their matrix-free stage, DGTD_KERNEL_VALU);
  * the only kernel of quadrilaterals (AUTO selects it there). */

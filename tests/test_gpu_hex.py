@@ -82,7 +82,7 @@ def test_hex_kernel_choice_positions_and_probes():
 
 @pytest.mark.parametrize("order", [1, 2, 3, 4, 5])
 def test_hex_matrix_free_matches_oracle(order):
-    """The matrix-free hexahedron stage (kernel "valu", hex_stage.hip)
+    """The matrix-free hexahedron stage (kernel "valu", tensor_stage.hip)
     against the oracle: every face code, random eps, mu, conductivity, both
     fluxes; FP64 to 1e-12, FP32 to 1e-5; and its RK4 / LSERK4 steps equal
     the assembled operator's to 1e-12."""
