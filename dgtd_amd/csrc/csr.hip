@@ -78,7 +78,7 @@ __global__ __launch_bounds__(256) void csr_stage(StageArgs<T> a)
     T own0 = T(0), own1 = T(0);
     auto load_own = [&]() {
         if constexpr (MODE == kModeLserk) {
-            own0 = a.res[r];
+            own0 = a.res_in ? a.res[r] : T(0);
             own1 = a.qin[r];
         } else if constexpr (MODE == kModeRk1) {
             own0 = a.qin[r];
@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void csr_stage(StageArgs<T> a)
         a.out[r] = rhs;
     } else if constexpr (MODE == kModeLserk) {
         const T rr = a.ca * own0 + a.dt * rhs;
-        a.res[r] = rr;
+        if (a.res_out) a.res[r] = rr;
         const T qn = own1 + a.cb * rr;
         a.out[r] = qn;
         check(qn);

@@ -40,7 +40,11 @@ __global__ __launch_bounds__(256) void dg_stage_kernel(StageArgs<T> a)
     extern __shared__ __align__(16) unsigned char smem_raw[];
     stage_load_ref<P, T>(a.mats, a.tabs, smem_raw);
     __syncthreads();
-    for (int blk = blockIdx.x; blk < a.nblk; blk += gridDim.x) stage_block<P, T, MODE, GLOBAL>(a, smem_raw, blk);
+    if (a.keep_out) {
+        for (int blk = blockIdx.x; blk < a.nblk; blk += gridDim.x) stage_block<P, T, MODE, GLOBAL, true>(a, smem_raw, blk);
+    } else {
+        for (int blk = blockIdx.x; blk < a.nblk; blk += gridDim.x) stage_block<P, T, MODE, GLOBAL, false>(a, smem_raw, blk);
+    }
 }
 
 template <int P, typename T, int MODE>
@@ -55,9 +59,11 @@ hipError_t launch_one(const StageArgs<T>& a, int grid, hipStream_t s)
 template <int P, typename T>
 hipError_t launch_mode(const StageArgs<T>& a, int mode, int grid, hipStream_t s)
 {
-    switch (mode) {
+    switch (lserk_mode(a, mode)) {
         case kModeMult: return launch_one<P, T, kModeMult>(a, grid, s);
         case kModeLserk: return launch_one<P, T, kModeLserk>(a, grid, s);
+        case kModeLserkFirst: return launch_one<P, T, kModeLserkFirst>(a, grid, s);
+        case kModeLserkLast: return launch_one<P, T, kModeLserkLast>(a, grid, s);
         case kModeRk1: return launch_one<P, T, kModeRk1>(a, grid, s);
         case kModeRk2: return launch_one<P, T, kModeRk2>(a, grid, s);
         case kModeRk3: return launch_one<P, T, kModeRk3>(a, grid, s);
@@ -83,6 +89,8 @@ int occupancy_one()
     constexpr size_t bytes = Smem<P, T>::bytes;
     set_smem_attr<P, T, kModeMult>();
     set_smem_attr<P, T, kModeLserk>();
+    set_smem_attr<P, T, kModeLserkFirst>();
+    set_smem_attr<P, T, kModeLserkLast>();
     set_smem_attr<P, T, kModeRk1>();
     set_smem_attr<P, T, kModeRk2>();
     set_smem_attr<P, T, kModeRk3>();

@@ -187,7 +187,8 @@ __global__ __launch_bounds__(256) void dg_tri_stage(StageArgs<T> a)
             T rv[6], xv[6];
 #pragma unroll
             for (int c = 0; c < 6; ++c) {
-                if constexpr (MODE == kModeLserk || MODE == kModeRk2 || MODE == kModeRk3 || MODE == kModeRk4)
+                if constexpr (MODE == kModeLserk || MODE == kModeLserkLast || MODE == kModeRk2 || MODE == kModeRk3 ||
+                              MODE == kModeRk4)
                     rv[c] = a.res[c * N + idx];
                 if constexpr (MODE == kModeRk2 || MODE == kModeRk3) xv[c] = a.x[c * N + idx];
             }
@@ -232,10 +233,11 @@ __global__ __launch_bounds__(256) void dg_tri_stage(StageArgs<T> a)
                 const T qv = sQ[c * EB * NP + el * NP + i];
                 if constexpr (MODE == kModeMult) {
                     a.out[o] = rhs[c];
-                } else if constexpr (MODE == kModeLserk) {
-                    const T r = a.ca * rv[c] + a.dt * rhs[c];
+                } else if constexpr (is_lserk(MODE)) {
+                    T r = a.dt * rhs[c];
+                    if constexpr (MODE != kModeLserkFirst) r = a.ca * rv[c] + r;
                     const T qn = qv + a.cb * r;
-                    a.res[o] = r;
+                    if constexpr (MODE != kModeLserkLast) a.res[o] = r;
                     a.out[o] = qn;
                     bad = bad || unstable_entry(qn);
                 } else if constexpr (MODE == kModeRk1) {
@@ -251,7 +253,7 @@ __global__ __launch_bounds__(256) void dg_tri_stage(StageArgs<T> a)
                 }
             }
         }
-        if constexpr (MODE == kModeLserk || MODE == kModeRk4) report_unstable(a.unstable, bad);
+        if constexpr (is_lserk(MODE) || MODE == kModeRk4) report_unstable(a.unstable, bad);
     }
 }
 
@@ -277,6 +279,8 @@ void tri_prepare_order()
 {
     tri_set_attr<P, T, kModeMult>();
     tri_set_attr<P, T, kModeLserk>();
+    tri_set_attr<P, T, kModeLserkFirst>();
+    tri_set_attr<P, T, kModeLserkLast>();
     tri_set_attr<P, T, kModeRk1>();
     tri_set_attr<P, T, kModeRk2>();
     tri_set_attr<P, T, kModeRk3>();
@@ -286,9 +290,11 @@ void tri_prepare_order()
 template <int P, typename T>
 hipError_t tri_launch_mode(const StageArgs<T>& a, int mode, int grid, hipStream_t s)
 {
-    switch (mode) {
+    switch (lserk_mode(a, mode)) {
         case kModeMult: return tri_launch_one<P, T, kModeMult>(a, grid, s);
         case kModeLserk: return tri_launch_one<P, T, kModeLserk>(a, grid, s);
+        case kModeLserkFirst: return tri_launch_one<P, T, kModeLserkFirst>(a, grid, s);
+        case kModeLserkLast: return tri_launch_one<P, T, kModeLserkLast>(a, grid, s);
         case kModeRk1: return tri_launch_one<P, T, kModeRk1>(a, grid, s);
         case kModeRk2: return tri_launch_one<P, T, kModeRk2>(a, grid, s);
         case kModeRk3: return tri_launch_one<P, T, kModeRk3>(a, grid, s);

@@ -21,7 +21,14 @@ enum StageMode : int {
     kModeRk2 = 3,    // k = L(y):  out(y') = x + ca k, res(z) += cb k
     kModeRk3 = 4,    // same as kModeRk2 with other coefficients
     kModeRk4 = 5,    // k = L(y):  out(x) = res(z) + ca k
+    // kModeLserk without the residual's read (res_in false) or store (res_out
+    // false): compile-time forms of the per-node kernels, where a run-time
+    // test around the accesses cost registers and waits (triangles order 4:
+    // FP32 126 -> 151 us, FP64 231 -> 389 us); chosen by lserk_mode
+    kModeLserkFirst = 6,
+    kModeLserkLast = 7,
 };
+constexpr bool is_lserk(int mode) { return mode == kModeLserk || mode == kModeLserkFirst || mode == kModeLserkLast; }
 
 template <typename T>
 struct StageArgs {
@@ -45,12 +52,29 @@ struct StageArgs {
     int64_t nrows, nnz;
     int np;  // nodes per element
     int* unstable;  // non-null: set to 1 when a stored state entry is unstable (unstable_entry)
+    // LSERK: whether the stage reads and leaves the residual.  The first stage
+    // of a step has ca = 0 and the next step starts afresh, so a step needs no
+    // residual read in its first stage and none stored by its last: 18
+    // passes over a state buffer per step instead of 20.
+    bool res_in, res_out;
+    // Whether the stage output is stored for reuse (else it streams past the
+    // caches): while the state, the output and the element records fit the 256
+    // MB Infinity Cache together, the next stage reads them from there.
+    // Triangles order 4 FP32, 106 MB per buffer: 126 -> 113 us per stage; 146
+    // MB and above lose 1-4 % (order-3 tetrahedra FP32 207 -> 210 us).
+    bool keep_out;
     // matrix-free Global operator on tetrahedra and triangles: the kernels'
     // Global variant (SMA faces, codes 3 and 6, upwinded fully whatever alpha;
     // conductivity) with sigma/eps_r per element in sig (NULL = none)
     bool global;
     const T* sig;
 };
+
+template <typename T>
+inline int lserk_mode(const StageArgs<T>& a, int mode)
+{
+    return mode != kModeLserk ? mode : !a.res_in ? kModeLserkFirst : !a.res_out ? kModeLserkLast : kModeLserk;
+}
 
 // Stability test of the reference's time loop (Solver::run, Solver.cpp:499-516,
 // flags a non-finite state norm or one above 1e20), applied to the entries a

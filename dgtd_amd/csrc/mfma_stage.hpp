@@ -282,7 +282,8 @@ __device__ MfmaLds<P, T, DIM> mfma_load_ref(const T* mats, const int* tabs, unsi
 
 // One wave-task: the fused stage of elements [task*8, task*8 + 8) of the mesh
 // described by `a`.  Only wave-level synchronisation inside.
-template <int P, typename T, int MODE, int DIM, int CFG>
+// KEEP: StageArgs::keep_out.
+template <int P, typename T, int MODE, int DIM, int CFG, bool KEEP = false>
 __device__ __forceinline__ void mfma_task(const StageArgs<T>& a, const MfmaLds<P, T, DIM>& L, const int task)
 {
     using S = MShape<P, DIM>;
@@ -483,7 +484,10 @@ __device__ __forceinline__ void mfma_task(const StageArgs<T>& a, const MfmaLds<P
         return (h ? 3 * nb_bytes : 0u) + (uint32_t)(tc - h * TE * NP) * SZ;
     };
     auto lin_soff = [&](int x) { return x * nb_bytes + (uint32_t)e0 * NP * SZ; };
-    const rsrc_t rres = make_rsrc(a.res, bytes);
+    // an LSERK stage that needs no residual reads (or stores) it through a
+    // descriptor of length 0: loads return 0, stores are dropped, no branch
+    const rsrc_t rres = make_rsrc(a.res, MODE != kModeLserk || a.res_in ? bytes : 0u);
+    const rsrc_t rres_out = make_rsrc(a.res, MODE != kModeLserk || a.res_out ? bytes : 0u);
     const rsrc_t rout = make_rsrc(a.out, bytes);
     const rsrc_t rx = make_rsrc(a.x, bytes);
     // the lane's linear slots, the same for every x: byte offsets (lane part)
@@ -670,24 +674,24 @@ __device__ __forceinline__ void mfma_task(const StageArgs<T>& a, const MfmaLds<P
             const uint32_t so = lin_soff(x);
             const T rhs = Sg[lst[k]];
             const T qv = U[lqv[k] + x * TE * US];
-            constexpr int nt = kAuxNontemporal;
+            constexpr int nt = kAuxNontemporal, keep = KEEP ? 0 : kAuxNontemporal;
             if constexpr (MODE == kModeMult) {
-                bstore<nt>(rhs, rout, vo, so);
+                bstore<keep>(rhs, rout, vo, so);
             } else if constexpr (MODE == kModeLserk) {
                 const T rr = a.ca * rl[cur][k] + a.dt * rhs;
                 const T qn = qv + a.cb * rr;
-                bstore<nt>(rr, rres, vo, so);
-                bstore<nt>(qn, rout, vo, so);
+                bstore<nt>(rr, rres_out, vo, so);
+                bstore<keep>(qn, rout, vo, so);
                 bad = bad || unstable_entry(qn);
             } else if constexpr (MODE == kModeRk1) {
-                bstore<nt>(qv + a.ca * rhs, rout, vo, so);
+                bstore<keep>(qv + a.ca * rhs, rout, vo, so);
                 bstore<nt>(qv + a.cb * rhs, rres, vo, so);
             } else if constexpr (MODE == kModeRk2 || MODE == kModeRk3) {
-                bstore<nt>(xl[cur][k] + a.ca * rhs, rout, vo, so);
+                bstore<keep>(xl[cur][k] + a.ca * rhs, rout, vo, so);
                 bstore<nt>(rl[cur][k] + a.cb * rhs, rres, vo, so);
             } else {
                 const T qn = rl[cur][k] + a.ca * rhs;
-                bstore<nt>(qn, rout, vo, so);
+                bstore<keep>(qn, rout, vo, so);
                 bad = bad || unstable_entry(qn);
             }
         }
@@ -713,8 +717,13 @@ __global__ __launch_bounds__((MWaves<P, T, DIM, CFG>::W * 64)) void dg_stage_mfm
     const int per_xcd = (ntasks + nxcd - 1) / nxcd;
     const int t_begin = xcd * per_xcd;
     const int t_end = min(ntasks, t_begin + per_xcd);
-    for (int tix = t_begin + bin * WAVES + wave; tix < t_end; tix += bpx * WAVES)
-        mfma_task<P, T, MODE, DIM, CFG>(a, L, a.order ? a.order[tix] : tix);
+    if (a.keep_out) {
+        for (int tix = t_begin + bin * WAVES + wave; tix < t_end; tix += bpx * WAVES)
+            mfma_task<P, T, MODE, DIM, CFG, true>(a, L, a.order ? a.order[tix] : tix);
+    } else {
+        for (int tix = t_begin + bin * WAVES + wave; tix < t_end; tix += bpx * WAVES)
+            mfma_task<P, T, MODE, DIM, CFG, false>(a, L, a.order ? a.order[tix] : tix);
+    }
 }
 
 // Batch variant: the running instances of element shape DIM and order P, one
@@ -754,6 +763,8 @@ __global__ __launch_bounds__((MWaves<P, T, DIM, CFG>::W * 64)) void dg_batch_sta
         a.geo = uniform(I.geo);
         a.conn = uniform(I.conn);
         a.unstable = b.stage == 4 ? &b.inst[inst].unstable : nullptr;  // the step's last stage
+        a.res_in = b.stage != 0;
+        a.res_out = b.stage != 4;
         mfma_task<P, T, kModeLserk, DIM, CFG>(a, L, blk);
     }
 }

@@ -59,7 +59,7 @@ __device__ __forceinline__ void stage_load_ref(const T* __restrict__ mats, const
 // GLOBAL: the Global operator's form of the same stage (GlobalEvolution.cpp:
 // 628-1088): SMA faces weighted as at alpha = 1 (DGOperatorFactory.h:485-495,
 // 587-591) and -sigma/eps E on the E rows (:1351-1361).
-template <int P, typename T, int MODE, bool GLOBAL = false>
+template <int P, typename T, int MODE, bool GLOBAL = false, bool KEEP = false>
 __device__ __forceinline__ void stage_block(const StageArgs<T>& a, unsigned char* smem_raw, int blk)
 {
     using S = Shape<P>;
@@ -190,7 +190,8 @@ __device__ __forceinline__ void stage_block(const StageArgs<T>& a, unsigned char
             T rv[6], xv[6];
 #pragma unroll
             for (int c = 0; c < 6; ++c) {
-                if constexpr (MODE == kModeLserk || MODE == kModeRk2 || MODE == kModeRk3 || MODE == kModeRk4)
+                if constexpr (MODE == kModeLserk || MODE == kModeLserkLast || MODE == kModeRk2 || MODE == kModeRk3 ||
+                              MODE == kModeRk4)
                     rv[c] = __builtin_nontemporal_load(a.res + c * N + idx);
                 if constexpr (MODE == kModeRk2 || MODE == kModeRk3) xv[c] = a.x[c * N + idx];
             }
@@ -232,28 +233,33 @@ __device__ __forceinline__ void stage_block(const StageArgs<T>& a, unsigned char
             for (int c = 0; c < 6; ++c) {
                 const size_t o = c * N + idx;
                 const T qv = sQ[c * EB * NP + el * NP + i];
+                auto store_out = [&](T v) {
+                    if constexpr (KEEP) a.out[o] = v;
+                    else __builtin_nontemporal_store(v, a.out + o);
+                };
                 if constexpr (MODE == kModeMult) {
-                    __builtin_nontemporal_store(rhs[c], a.out + o);
-                } else if constexpr (MODE == kModeLserk) {
-                    const T r = a.ca * rv[c] + a.dt * rhs[c];
+                    store_out(rhs[c]);
+                } else if constexpr (is_lserk(MODE)) {
+                    T r = a.dt * rhs[c];
+                    if constexpr (MODE != kModeLserkFirst) r = a.ca * rv[c] + r;
                     const T qn = qv + a.cb * r;
-                    __builtin_nontemporal_store(r, a.res + o);
-                    __builtin_nontemporal_store(qn, a.out + o);
+                    if constexpr (MODE != kModeLserkLast) __builtin_nontemporal_store(r, a.res + o);
+                    store_out(qn);
                     bad = bad || unstable_entry(qn);
                 } else if constexpr (MODE == kModeRk1) {
-                    __builtin_nontemporal_store(qv + a.ca * rhs[c], a.out + o);
+                    store_out(qv + a.ca * rhs[c]);
                     __builtin_nontemporal_store(qv + a.cb * rhs[c], a.res + o);
                 } else if constexpr (MODE == kModeRk2 || MODE == kModeRk3) {
-                    __builtin_nontemporal_store(xv[c] + a.ca * rhs[c], a.out + o);
+                    store_out(xv[c] + a.ca * rhs[c]);
                     __builtin_nontemporal_store(rv[c] + a.cb * rhs[c], a.res + o);
                 } else {  // kModeRk4
                     const T qn = rv[c] + a.ca * rhs[c];
-                    __builtin_nontemporal_store(qn, a.out + o);
+                    store_out(qn);
                     bad = bad || unstable_entry(qn);
                 }
             }
         }
-        if constexpr (MODE == kModeLserk || MODE == kModeRk4) report_unstable(a.unstable, bad);
+        if constexpr (is_lserk(MODE) || MODE == kModeRk4) report_unstable(a.unstable, bad);
     }
     __syncthreads();  // LDS tiles free for the next block
 }

@@ -137,8 +137,9 @@ __global__ __launch_bounds__(kThreads) void tensor_stage(StageArgs<T> a)
     // the update's operands, in flight until the end
     constexpr bool kNeedRes = MODE != kModeMult && MODE != kModeRk1;
     constexpr bool kNeedX = MODE == kModeRk2 || MODE == kModeRk3;
-    v4 rv, xv;
-    if constexpr (kNeedRes) rv = load(a.res);
+    v4 rv = {T(0), T(0), T(0), T(0)}, xv;
+    if constexpr (kNeedRes)
+        if (MODE != kModeLserk || a.res_in) rv = load(a.res);
     if constexpr (kNeedX) xv = load(a.x);
 #pragma unroll
     for (int r = 0; r < 4; ++r) sq[c0 * NE + first + r] = q[r];
@@ -273,14 +274,17 @@ __global__ __launch_bounds__(kThreads) void tensor_stage(StageArgs<T> a)
         if constexpr (MODE == kModeLserk || MODE == kModeRk4) bad = bad || (first + r < cnt && unstable_entry(o[r]));
     }
     constexpr bool kRes = MODE != kModeMult && MODE != kModeRk4;
+    const bool keep = MODE != kModeLserk || a.res_out;
     if (full) {
-        if constexpr (kRes) *reinterpret_cast<v4*>(a.res + off + first) = r2;
+        if constexpr (kRes)
+            if (keep) *reinterpret_cast<v4*>(a.res + off + first) = r2;
         *reinterpret_cast<v4*>(a.out + off + first) = o;
     } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
             if (first + r < cnt) {
-                if constexpr (kRes) a.res[off + first + r] = r2[r];
+                if constexpr (kRes)
+                    if (keep) a.res[off + first + r] = r2[r];
                 a.out[off + first + r] = o[r];
             }
     }
