@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "dgtd_hip.h"
+#include "host_copy.hpp"
 #include "kernels.hpp"
 #include "trace.hpp"
 #include "mesh.hpp"
@@ -83,6 +84,7 @@ struct dgtd_batch {
     // dgtd_batch_add does its host setup and upload outside it, so callers may
     // admit from worker threads while another thread steps the batch.
     std::mutex mu;
+    dgtd::HostCopy host_copy;  // used with mu held
     int device = 0, precision = 32;
     double alpha = 1.0;
     int max_slots = 0;
@@ -807,13 +809,9 @@ int dgtd_batch_get_state(dgtd_batch* b, int32_t id, double* x)
         if (s.state == dgtd::kSlotFree || s.state == dgtd_batch::kSlotReserved)
             return dgtd::api_fail(DGTD_E_STATE, "instance slot is free or still being set up");
         const size_t ndofs = 6 * (size_t)nodes(s.dim, s.order) * s.K;
-        if (b->precision == 64) {
-            hcheck(hipMemcpy(x, s.buf[s.cur], sizeof(double) * ndofs, hipMemcpyDeviceToHost), "D2H state");
-        } else {
-            std::vector<float> tmp(ndofs);
-            hcheck(hipMemcpy(tmp.data(), s.buf[s.cur], sizeof(float) * ndofs, hipMemcpyDeviceToHost), "D2H state");
-            std::copy(tmp.begin(), tmp.end(), x);
-        }
+        hcheck(b->precision == 64 ? b->host_copy.to_host(static_cast<const double*>(s.buf[s.cur]), x, ndofs, b->stream)
+                                  : b->host_copy.to_host(static_cast<const float*>(s.buf[s.cur]), x, ndofs, b->stream),
+               "D2H state");
     } catch (const std::exception& e) {
         return batch_error(e);
     }

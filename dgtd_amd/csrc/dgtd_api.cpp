@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "fields.hpp"
+#include "host_copy.hpp"
 #include "kernels.hpp"
 #include "trace.hpp"
 #include "tensor_dev.hpp"
@@ -519,30 +520,20 @@ struct dgtd_op {
         tfsf<T>(tm, static_cast<T*>(out), 1.0, nullptr, 0.0, s);
     }
 
+    dgtd::HostCopy host_copy;
+
     void to_device(const double* h, void* d)
     {
-        if (precision == 64) {
-            hip_check(hipMemcpyAsync(d, h, sizeof(double) * ndofs, hipMemcpyHostToDevice, stream), "H2D");
-        } else {
-            std::vector<float> tmp(h, h + ndofs);
-            hip_check(hipMemcpyAsync(d, tmp.data(), sizeof(float) * ndofs, hipMemcpyHostToDevice, stream),
-                      "H2D");
-            hip_check(hipStreamSynchronize(stream), "sync");
-        }
+        hip_check(precision == 64 ? host_copy.to_device(h, static_cast<double*>(d), ndofs, stream)
+                                  : host_copy.to_device(h, static_cast<float*>(d), ndofs, stream),
+                  "H2D");
     }
 
     void to_host(const void* d, double* h)
     {
-        if (precision == 64) {
-            hip_check(hipMemcpyAsync(h, d, sizeof(double) * ndofs, hipMemcpyDeviceToHost, stream), "D2H");
-            hip_check(hipStreamSynchronize(stream), "sync");
-        } else {
-            std::vector<float> tmp(ndofs);
-            hip_check(hipMemcpyAsync(tmp.data(), d, sizeof(float) * ndofs, hipMemcpyDeviceToHost, stream),
-                      "D2H");
-            hip_check(hipStreamSynchronize(stream), "sync");
-            std::copy(tmp.begin(), tmp.end(), h);
-        }
+        hip_check(precision == 64 ? host_copy.to_host(static_cast<const double*>(d), h, ndofs, stream)
+                                  : host_copy.to_host(static_cast<const float*>(d), h, ndofs, stream),
+                  "D2H");
     }
 };
 
