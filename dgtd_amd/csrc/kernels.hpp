@@ -313,6 +313,10 @@ inline int norms_tile(int Np)
 constexpr int kNormsMaxParts = 1024;
 hipError_t norms_scratch(int device, double** ptr);
 
+// Fills p with values in [-1, 1) (the autotuner's test state).
+template <typename T>
+hipError_t launch_fill_noise(T* p, int64_t n, hipStream_t s);
+
 template <typename T>
 hipError_t launch_norms(const T* q, int K, int Np, const double* Mref, const double* jac,
                         const double* eps, const double* mu, double* partials, int nparts,

@@ -149,6 +149,18 @@ template hipError_t launch_norms<float>(const float*, int, int, const double*, c
 // Point probes: one wave per (probe, component) forms
 // sum_n w[probe][n] * q[c*N + elem[probe]*Np + n] in FP64; probes outside
 // the mesh (elem < 0) give NaN.
+// p[i] in [-1, 1), from a mixed counter (the finalising steps of MurmurHash3).
+template <typename T>
+__global__ __launch_bounds__(kThreads) void fill_noise(T* p, int64_t n)
+{
+    for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) {
+        uint32_t h = (uint32_t)i * 0x9e3779b9u;
+        h = (h ^ (h >> 16)) * 0x85ebca6bu;
+        h = (h ^ (h >> 13)) * 0xc2b2ae35u;
+        p[i] = (T)(int32_t)(h ^ (h >> 16)) * T(1.0 / 2147483648.0);
+    }
+}
+
 template <typename T>
 __global__ __launch_bounds__(64) void probe_sample(const T* __restrict__ q, size_t N, int Np,
                                                    const int* __restrict__ elem,
@@ -176,5 +188,15 @@ template hipError_t launch_probe_sample<double>(const double*, size_t, int, int,
                                                 double*, hipStream_t);
 template hipError_t launch_probe_sample<float>(const float*, size_t, int, int, const int*, const double*,
                                                double*, hipStream_t);
+
+template <typename T>
+hipError_t launch_fill_noise(T* p, int64_t n, hipStream_t s)
+{
+    const int64_t blocks = (n + kThreads - 1) / kThreads;
+    hipLaunchKernelGGL(fill_noise<T>, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(kThreads), 0, s, p, n);
+    return hipGetLastError();
+}
+template hipError_t launch_fill_noise<double>(double*, int64_t, hipStream_t);
+template hipError_t launch_fill_noise<float>(float*, int64_t, hipStream_t);
 
 }  // namespace dgtd

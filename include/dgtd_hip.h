@@ -286,8 +286,8 @@ int dgtd_op_last_kernel_us(const dgtd_op* op, double* avg_us, int32_t* launches)
 int dgtd_op_kernel_variant(const dgtd_op* op, int32_t* variant);
 
 /* The stage kernel the autotuner chose (no counterpart in the reference).
- * With DGTD_KERNEL_AUTO every candidate is timed at create on the zeroed
- * state (the fused LSERK stage for LSERK4 operators, Mult otherwise; two
+ * With DGTD_KERNEL_AUTO every candidate is timed at create on noise
+ * (the fused LSERK stage for LSERK4 operators, Mult otherwise; two
  * rounds, three launches then about 1 ms of launches each, the lower mean
  * kept) and the fastest kept; the choice is
  * cached for the process per (element shape, order, precision, stage mode,
