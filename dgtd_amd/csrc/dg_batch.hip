@@ -17,6 +17,14 @@ namespace {
 
 using namespace valu;
 
+template <int P, typename T>
+__device__ __forceinline__ void batch_block(const StageArgs<T>& a, unsigned char* smem_raw, int blk)
+{
+    Fetched<P, T> f;
+    stage_fetch<P, T>(a, blk, f);
+    stage_block<P, T, kModeLserk>(a, smem_raw, blk, f);
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void dg_batch_stage(BatchArgs<T> b)
 {
@@ -55,12 +63,13 @@ __global__ __launch_bounds__(256) void dg_batch_stage(BatchArgs<T> b)
         a.conn = I.conn;
         a.unstable = b.stage == 4 ? &b.inst[w.inst].unstable : nullptr;  // the step's last stage
         switch (order) {
-            case 1: stage_block<1, T, kModeLserk>(a, smem_raw, w.blk); break;
-            case 2: stage_block<2, T, kModeLserk>(a, smem_raw, w.blk); break;
-            case 3: stage_block<3, T, kModeLserk>(a, smem_raw, w.blk); break;
-            case 4: stage_block<4, T, kModeLserk>(a, smem_raw, w.blk); break;
-            default: stage_block<5, T, kModeLserk>(a, smem_raw, w.blk); break;
+            case 1: batch_block<1, T>(a, smem_raw, w.blk); break;
+            case 2: batch_block<2, T>(a, smem_raw, w.blk); break;
+            case 3: batch_block<3, T>(a, smem_raw, w.blk); break;
+            case 4: batch_block<4, T>(a, smem_raw, w.blk); break;
+            default: batch_block<5, T>(a, smem_raw, w.blk); break;
         }
+        __syncthreads();  // LDS tiles free for the next block
     }
 }
 

@@ -37,30 +37,80 @@ struct Smem {
 // Threads per block of the per-node kernels (single-mesh and batch).
 constexpr int kThreads = 256;
 
+// A block's fields and records on their way from memory into LDS.
+template <int P, typename T>
+struct Fetched {
+    using S = Shape<P>;
+    static constexpr int NG = (S::EB * kGeoStrideDev + kThreads - 1) / kThreads;
+    static constexpr int NC = (S::EB * kConnStrideDev + kThreads - 1) / kThreads;
+    T q[6], g[NG];
+    int c[NC];
+};
+
+// Issues every load of element block blk's fields and records (threads past
+// the end load a clamped, valid address).
+template <int P, typename T>
+__device__ __forceinline__ void stage_fetch(const StageArgs<T>& a, int blk, Fetched<P, T>& f)
+{
+    using S = Shape<P>;
+    constexpr int NP = S::NP, EB = S::EB;
+    const int tid = threadIdx.x;
+    const size_t N = (size_t)NP * a.K;
+    const int e0 = blk * EB;
+    const int ne = min(EB, a.K - e0);
+    const size_t base = (size_t)e0 * NP;
+    const int cnt = ne * NP, ng = ne * kGeoStrideDev, nc = ne * kConnStrideDev;
+    const int iq = tid < cnt ? tid : cnt - 1;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) f.q[c] = a.qin[c * N + base + iq];
+#pragma unroll
+    for (int k = 0; k < Fetched<P, T>::NG; ++k) {
+        const int i = tid + k * kThreads;
+        f.g[k] = a.geo[(size_t)e0 * kGeoStrideDev + (i < ng ? i : ng - 1)];
+    }
+#pragma unroll
+    for (int k = 0; k < Fetched<P, T>::NC; ++k) {
+        const int i = tid + k * kThreads;
+        f.c[k] = a.conn[(size_t)e0 * kConnStrideDev + (i < nc ? i : nc - 1)];
+    }
+}
+
 // Loads the order-P reference matrices and tables into LDS (block-wide;
-// the caller synchronises before use), several loads in flight per thread
-// (up to 55 values per thread at order 5).
+// stage_block's first barrier follows).  The tables' loads are issued before
+// the matrices', of which several are in flight per thread (up to 55 values
+// per thread at order 5), so one memory latency covers both.
 template <int P, typename T>
 __device__ __forceinline__ void stage_load_ref(const T* __restrict__ mats, const int* __restrict__ tabs,
                                                unsigned char* smem_raw)
 {
     using S = Shape<P>;
     using L = Smem<P, T>;
-    constexpr int NFP = S::NFP, EB = S::EB;
+    constexpr int NT = 4 * S::NFP + 96 * S::NFP, NTT = (NT + kThreads - 1) / kThreads;
     T* sD = reinterpret_cast<T*>(smem_raw);
-    int* sFm = reinterpret_cast<int*>(sD + L::nReal) + EB * kConnStrideDev;
-    lds_copy<8>(sD, mats, L::nD + L::nL, (int)threadIdx.x, kThreads);
-    lds_copy<8>(sFm, tabs, 4 * NFP + 96 * NFP, (int)threadIdx.x, kThreads);
+    int* sFm = reinterpret_cast<int*>(sD + L::nReal) + S::EB * kConnStrideDev;
+    const int tid = threadIdx.x;
+    int tv[NTT];
+#pragma unroll
+    for (int k = 0; k < NTT; ++k) {
+        const int i = tid + k * kThreads;
+        tv[k] = tabs[i < NT ? i : NT - 1];
+    }
+    lds_copy<8>(sD, mats, L::nD + L::nL, tid, kThreads);
+#pragma unroll
+    for (int k = 0; k < NTT; ++k)
+        if (tid + k * kThreads < NT) sFm[tid + k * kThreads] = tv[k];
 }
 
-// One element block (EB elements from e0 = blk*EB) of one stage: gather,
-// flux, curl, LIFT and the stage update.  Starts and ends with a block-wide
-// barrier; the reference matrices must already be in LDS.
+// One element block (EB elements from e0 = blk*EB, fetched in f) of one stage:
+// gather, flux, curl, LIFT and the stage update.  The reference matrices are in
+// LDS or on their way there (its first barrier waits for them); the caller puts
+// a block-wide barrier between two element blocks.
 // GLOBAL: the Global operator's form of the same stage (GlobalEvolution.cpp:
 // 628-1088): SMA faces weighted as at alpha = 1 (DGOperatorFactory.h:485-495,
 // 587-591) and -sigma/eps E on the E rows (:1351-1361).
 template <int P, typename T, int MODE, bool GLOBAL = false, bool KEEP = false>
-__device__ __forceinline__ void stage_block(const StageArgs<T>& a, unsigned char* smem_raw, int blk)
+__device__ __forceinline__ void stage_block(const StageArgs<T>& a, unsigned char* smem_raw, int blk,
+                                            const Fetched<P, T>& fetched)
 {
     using S = Shape<P>;
     using L = Smem<P, T>;
@@ -81,39 +131,18 @@ __device__ __forceinline__ void stage_block(const StageArgs<T>& a, unsigned char
     {
         const int e0 = blk * EB;
         const int ne = min(EB, K - e0);
-        __syncthreads();  // previous iteration finished with sQ/sF/sG/sC (and tables loaded)
         {
-            // every load of the block's fields and records in flight, then the
-            // LDS writes (out-of-range threads load a clamped, valid address)
-            constexpr int NG = (EB * kGeoStrideDev + kThreads - 1) / kThreads;
-            constexpr int NC = (EB * kConnStrideDev + kThreads - 1) / kThreads;
-            const size_t base = (size_t)e0 * NP;
             const int cnt = ne * NP, ng = ne * kGeoStrideDev, nc = ne * kConnStrideDev;
-            const int iq = tid < cnt ? tid : cnt - 1;
-            T q[6], gv[NG];
-            int cv[NC];
-#pragma unroll
-            for (int c = 0; c < 6; ++c) q[c] = a.qin[c * N + base + iq];
-#pragma unroll
-            for (int k = 0; k < NG; ++k) {
-                const int i = tid + k * kThreads;
-                gv[k] = a.geo[(size_t)e0 * kGeoStrideDev + (i < ng ? i : ng - 1)];
-            }
-#pragma unroll
-            for (int k = 0; k < NC; ++k) {
-                const int i = tid + k * kThreads;
-                cv[k] = a.conn[(size_t)e0 * kConnStrideDev + (i < nc ? i : nc - 1)];
-            }
             if (tid < cnt) {
 #pragma unroll
-                for (int c = 0; c < 6; ++c) sQ[c * EB * NP + tid] = q[c];
+                for (int c = 0; c < 6; ++c) sQ[c * EB * NP + tid] = fetched.q[c];
             }
 #pragma unroll
-            for (int k = 0; k < NG; ++k)
-                if (tid + k * kThreads < ng) sG[tid + k * kThreads] = gv[k];
+            for (int k = 0; k < Fetched<P, T>::NG; ++k)
+                if (tid + k * kThreads < ng) sG[tid + k * kThreads] = fetched.g[k];
 #pragma unroll
-            for (int k = 0; k < NC; ++k)
-                if (tid + k * kThreads < nc) sC[tid + k * kThreads] = cv[k];
+            for (int k = 0; k < Fetched<P, T>::NC; ++k)
+                if (tid + k * kThreads < nc) sC[tid + k * kThreads] = fetched.c[k];
         }
         __syncthreads();
 
@@ -261,7 +290,6 @@ __device__ __forceinline__ void stage_block(const StageArgs<T>& a, unsigned char
         }
         if constexpr (is_lserk(MODE) || MODE == kModeRk4) report_unstable(a.unstable, bad);
     }
-    __syncthreads();  // LDS tiles free for the next block
 }
 
 }  // namespace valu
