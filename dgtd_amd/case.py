@@ -117,7 +117,7 @@ class Case:
         return x
 
     def needs_assembled_operator(self):
-        """True when kernel "auto" runs the assembled operator ("csr"), as the
+        """True when kernel "auto" runs the Global operator ("csr"), as the
         launcher decides: conductive materials, SMA faces (boundary or
         interior) with alpha != 1 under the Global or Maxwell operator (which
         weight SMA faces as at alpha = 1), quadrilateral meshes.  Hexahedral
@@ -130,7 +130,7 @@ class Case:
         return self.sigma is not None or global_sma or self.quads
 
     def operator(self, precision=64, integrator="rk4", kernel="auto", device=0):
-        """The case's operator; kernel="auto" selects the assembled one ("csr")
+        """The case's operator; kernel="auto" selects the Global one ("csr")
         where needs_assembled_operator() says so."""
         if kernel == "auto" and self.needs_assembled_operator():
             kernel = "csr"

@@ -220,7 +220,7 @@ void read_model(const dgtd::Json& c, const std::string& case_path, dgtd_case& cs
     // materials by element attribute (driver.cpp:946-966); the operator
     // applies eps_r, mu_r per element as 1/eps, 1/mu on the rhs, and the bulk
     // conductivity, normalised sigma_SI * Z0 (driver.cpp:962-963,
-    // PhysicalConstants.h:9-15), as -sigma/eps E (assembled operator only)
+    // PhysicalConstants.h:9-15), as -sigma/eps E (Global operator only)
     constexpr double kZ0 = 4.0e-7 * M_PI * 299792458.0;
     std::map<int, std::array<double, 3>> mat;
     if (!m.contains("materials")) throw std::runtime_error("JSON data does not include 'materials'.");

@@ -10,7 +10,7 @@
 //
 //   dgtd_launch CASE.json [--precision 64|32] [--integrator rk4|lserk4]
 //               [--kernel auto|valu|mfma|csr] [--final-time T] [--out DIR]
-// A case with conductive materials runs on the assembled operator (csr) under
+// A case with conductive materials runs on the Global operator (csr) under
 // --kernel auto.
 #include <chrono>
 #include <cmath>
@@ -102,7 +102,7 @@ int main(int argc, char** argv)
     o.precision = precision;
     o.integrator = integrator;
     // conductivity, or the Global operator's own SMA weighting (alpha != 1
-    // with SMA faces), needs the assembled operator
+    // with SMA faces), needs the Global operator
     bool sma = false;
     const int nfaces = mesh.nvert == 8 ? 6 : mesh.dim == 2 && mesh.nvert != 4 ? 3 : 4;
     for (int64_t i = 0; i < (int64_t)mesh.K * nfaces; ++i)

@@ -395,7 +395,7 @@ typedef struct {
     int32_t K, nv, order;
     double alpha, time_step, final_time, cfl;
     int32_t evolution_operator;   /* as named in the case (DGTD_OPERATOR_*; "global" when absent):
-                                   * the matrix-free hesthaven operator, or the assembled one
+                                   * the hesthaven operator, or the Global one
                                    * for conductivity, SMA faces with alpha != 1 under Global
                                    * or Maxwell, quadrilaterals and hexahedra */
     int32_t nsources, nprobes;
@@ -407,7 +407,7 @@ typedef struct {
     int32_t dim;                  /* 3: tetrahedral or hexahedral mesh; 2: triangle or
                                    * quadrilateral mesh (dgtd_case_mesh sets nvert = 4 for
                                    * quadrilaterals, 8 for hexahedra, which run on the
-                                   * assembled operator; such a case naming the hesthaven
+                                   * Global operator; such a case naming the hesthaven
                                    * operator is refused) */
     int32_t nfield_probes;        /* probes.field entries */
 } dgtd_case_info;
@@ -497,7 +497,7 @@ int dgtd_batch_footprint(const dgtd_mesh_desc* mesh, int32_t precision, int64_t*
  * matrix-core stage, order-1 tetrahedra on the per-node stage.  Conductivity
  * and state buffers of 4 GiB or more are refused (DGTD_E_UNSUPPORTED), and so
  * are quadrilateral and hexahedral meshes (nvert 4 with dim 2, nvert 8: the
- * assembled operator only); TF/SF
+ * Global operator only); TF/SF
  * faces (code 7) inject nothing without plane waves (dgtd_batch_add_tfsf). */
 int dgtd_batch_add(dgtd_batch* b, const dgtd_mesh_desc* mesh, const double* x0, double dt,
                    double final_time, int32_t* id);
@@ -560,7 +560,7 @@ int dgtd_mesh_vmaps(const dgtd_mesh_desc* mesh, double alpha, int32_t* vmapM, in
  * (DGTD_E_UNSUPPORTED otherwise). */
 int dgtd_mesh_geometry(const dgtd_mesh_desc* mesh, double alpha, double* geo);
 
-/* The assembled operator DGTD_KERNEL_CSR uploads, on the host in FP64 (the
+/* The operator DGTD_KERNEL_CSR applies, assembled on the host in FP64 (the
  * Global operator's matrix, DGOperatorFactory::buildGlobalOperator,
  * DGOperatorFactory.h:1428-1600): ndofs x ndofs CSR, rows and columns in the
  * state layout, mesh->sigma included.  Call with rowptr, col and val NULL to
