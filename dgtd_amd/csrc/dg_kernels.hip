@@ -39,52 +39,67 @@ using namespace valu;
 // three on a mesh of a block or two per CU (order 3 FP64, 48 / 3,072
 // tetrahedra: 8.7 -> 8.2 and 10.2 -> 9.8 us per stage; order 1 FP32, 1,296:
 // 5.4 -> 5.2 us; order 3 FP32, 24,576: 23.3 -> 22.1 us).
-template <int P, typename T, int MODE, bool GLOBAL, bool KEEP>
+template <int P, typename T, int MODE, bool GLOBAL, bool KEEP, bool SMALL>
 __device__ __forceinline__ void stage_blocks(const StageArgs<T>& a, unsigned char* smem_raw)
 {
     int blk = blockIdx.x;
     if (blk >= a.nblk) return;
-    Fetched<P, T> f;
-    stage_fetch<P, T>(a, blk, f);
-    stage_load_ref<P, T>(a.mats, a.tabs, smem_raw);
+    Fetched<P, T, SMALL> f;
+    stage_fetch<P, T, SMALL>(a, blk, f);
+    stage_load_ref<P, T, SMALL>(a.mats, a.tabs, smem_raw);
     for (;;) {
-        stage_block<P, T, MODE, GLOBAL, KEEP>(a, smem_raw, blk, f);
+        stage_block<P, T, MODE, GLOBAL, KEEP, SMALL>(a, smem_raw, blk, f);
         blk += gridDim.x;
         if (blk >= a.nblk) break;
         __syncthreads();  // LDS tiles free for the next block
-        stage_fetch<P, T>(a, blk, f);
+        stage_fetch<P, T, SMALL>(a, blk, f);
     }
 }
 
-template <int P, typename T, int MODE, bool GLOBAL>
+template <int P, typename T, int MODE, bool GLOBAL, bool SMALL>
 __global__ __launch_bounds__(256) void dg_stage_kernel(StageArgs<T> a)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    if (a.keep_out) stage_blocks<P, T, MODE, GLOBAL, true>(a, smem_raw);
-    else stage_blocks<P, T, MODE, GLOBAL, false>(a, smem_raw);
+    if (!SMALL && a.keep_out) stage_blocks<P, T, MODE, GLOBAL, true, SMALL>(a, smem_raw);
+    else stage_blocks<P, T, MODE, GLOBAL, false, SMALL>(a, smem_raw);
+}
+
+// A mesh of small blocks is far below the state size from which the shortened
+// LSERK4 stages are used, so those have no SMALL form.
+template <int MODE>
+constexpr bool has_small() { return MODE != kModeLserkFirst && MODE != kModeLserkLast; }
+
+template <int P, typename T, int MODE, bool SMALL>
+hipError_t launch_one(const StageArgs<T>& a, int grid, hipStream_t s)
+{
+    if constexpr (SMALL && !has_small<MODE>()) {
+        return hipErrorInvalidValue;
+    } else {
+        constexpr size_t bytes = Smem<P, T, SMALL>::bytes;
+        auto kern = a.global ? dg_stage_kernel<P, T, MODE, true, SMALL> : dg_stage_kernel<P, T, MODE, false, SMALL>;
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), bytes, s, a);
+        return hipGetLastError();
+    }
 }
 
 template <int P, typename T, int MODE>
-hipError_t launch_one(const StageArgs<T>& a, int grid, hipStream_t s)
+hipError_t launch_size(const StageArgs<T>& a, int grid, hipStream_t s)
 {
-    constexpr size_t bytes = Smem<P, T>::bytes;
-    auto kern = a.global ? dg_stage_kernel<P, T, MODE, true> : dg_stage_kernel<P, T, MODE, false>;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), bytes, s, a);
-    return hipGetLastError();
+    return a.small_blocks ? launch_one<P, T, MODE, true>(a, grid, s) : launch_one<P, T, MODE, false>(a, grid, s);
 }
 
 template <int P, typename T>
 hipError_t launch_mode(const StageArgs<T>& a, int mode, int grid, hipStream_t s)
 {
     switch (lserk_mode(a, mode)) {
-        case kModeMult: return launch_one<P, T, kModeMult>(a, grid, s);
-        case kModeLserk: return launch_one<P, T, kModeLserk>(a, grid, s);
-        case kModeLserkFirst: return launch_one<P, T, kModeLserkFirst>(a, grid, s);
-        case kModeLserkLast: return launch_one<P, T, kModeLserkLast>(a, grid, s);
-        case kModeRk1: return launch_one<P, T, kModeRk1>(a, grid, s);
-        case kModeRk2: return launch_one<P, T, kModeRk2>(a, grid, s);
-        case kModeRk3: return launch_one<P, T, kModeRk3>(a, grid, s);
-        case kModeRk4: return launch_one<P, T, kModeRk4>(a, grid, s);
+        case kModeMult: return launch_size<P, T, kModeMult>(a, grid, s);
+        case kModeLserk: return launch_size<P, T, kModeLserk>(a, grid, s);
+        case kModeLserkFirst: return launch_size<P, T, kModeLserkFirst>(a, grid, s);
+        case kModeLserkLast: return launch_size<P, T, kModeLserkLast>(a, grid, s);
+        case kModeRk1: return launch_size<P, T, kModeRk1>(a, grid, s);
+        case kModeRk2: return launch_size<P, T, kModeRk2>(a, grid, s);
+        case kModeRk3: return launch_size<P, T, kModeRk3>(a, grid, s);
+        case kModeRk4: return launch_size<P, T, kModeRk4>(a, grid, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -92,9 +107,13 @@ hipError_t launch_mode(const StageArgs<T>& a, int mode, int grid, hipStream_t s)
 template <int P, typename T, int MODE>
 void set_smem_attr()
 {
-    for (const void* kern : {reinterpret_cast<const void*>(dg_stage_kernel<P, T, MODE, false>),
-                             reinterpret_cast<const void*>(dg_stage_kernel<P, T, MODE, true>)})
+    for (const void* kern : {reinterpret_cast<const void*>(dg_stage_kernel<P, T, MODE, false, false>),
+                             reinterpret_cast<const void*>(dg_stage_kernel<P, T, MODE, true, false>)})
         (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Smem<P, T>::bytes);
+    if constexpr (has_small<MODE>())
+        for (const void* kern : {reinterpret_cast<const void*>(dg_stage_kernel<P, T, MODE, false, true>),
+                                 reinterpret_cast<const void*>(dg_stage_kernel<P, T, MODE, true, true>)})
+            (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Smem<P, T, true>::bytes);
 }
 
 // Raises the dynamic-LDS limit of every stage variant of this order (needed
@@ -112,7 +131,7 @@ int occupancy_one()
     set_smem_attr<P, T, kModeRk2>();
     set_smem_attr<P, T, kModeRk3>();
     set_smem_attr<P, T, kModeRk4>();
-    auto kern = dg_stage_kernel<P, T, kModeLserk, false>;
+    auto kern = dg_stage_kernel<P, T, kModeLserk, false, false>;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, 256, bytes) != hipSuccess) return 1;
     return nb > 0 ? nb : 1;
 }
@@ -145,14 +164,14 @@ int stage_blocks_per_cu(int order)
     }
 }
 
-int elements_per_block(int order)
+int elements_per_block(int order, bool small)
 {
     switch (order) {
-        case 1: return Shape<1>::EB;
-        case 2: return Shape<2>::EB;
-        case 3: return Shape<3>::EB;
-        case 4: return Shape<4>::EB;
-        case 5: return Shape<5>::EB;
+        case 1: return small ? Shape<1, true>::EB : Shape<1>::EB;
+        case 2: return small ? Shape<2, true>::EB : Shape<2>::EB;
+        case 3: return small ? Shape<3, true>::EB : Shape<3>::EB;
+        case 4: return small ? Shape<4, true>::EB : Shape<4>::EB;
+        case 5: return small ? Shape<5, true>::EB : Shape<5>::EB;
         default: return 1;
     }
 }

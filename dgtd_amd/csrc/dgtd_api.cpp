@@ -202,6 +202,7 @@ struct dgtd_op {
     double last_us = 0.0;
     int last_launches = 0;
 
+    bool small_blocks = false;  // StageArgs::small_blocks
     int64_t record_bytes = 0;  // geometry and connectivity records of the stage kernels
 
     // Below 12 MB per state buffer a stage runs from the L2s: the shortened
@@ -235,6 +236,7 @@ struct dgtd_op {
         dgtd::StageArgs<T> a{};
         a.K = K;
         a.nblk = nblk;
+        a.small_blocks = small_blocks;
         a.alpha = (T)alpha;
         a.res_in = a.res_out = true;
         // Infinity Cache: 256 MB, less a margin
@@ -1150,7 +1152,11 @@ int dgtd_op_create(const dgtd_mesh_desc* mesh, const dgtd_opts* opts, dgtd_op** 
         hip_check(hipStreamSynchronize(op->stream), "sync");
         hipDeviceProp_t prop;
         hip_check(hipGetDeviceProperties(&prop, op->device), "hipGetDeviceProperties");
-        const int epb = dgtd::elements_per_block(op->R.p);
+        // small element blocks while each of them has a CU to itself
+        // (stage_body.hpp, Shape)
+        const int epb_small = dgtd::elements_per_block(op->R.p, true);
+        op->small_blocks = op->K <= prop.multiProcessorCount * epb_small;
+        const int epb = op->small_blocks ? epb_small : dgtd::elements_per_block(op->R.p);
         op->nblk = (op->K + epb - 1) / epb;
         op->grid = std::max(1, std::min(op->nblk, prop.multiProcessorCount * bpc));
         bool any_mfma = false;

@@ -63,6 +63,9 @@ struct StageArgs {
     // Triangles order 4 FP32, 106 MB per buffer: 126 -> 113 us per stage; 146
     // MB and above lose 1-4 % (order-3 tetrahedra FP32 207 -> 210 us).
     bool keep_out;
+    // Per-node stage of tetrahedra: element blocks of half the size (nblk
+    // counts those; Shape in stage_body.hpp).
+    bool small_blocks;
     // matrix-free Global operator on tetrahedra and triangles: the kernels'
     // Global variant (SMA faces, codes 3 and 6, upwinded fully whatever alpha;
     // conductivity) with sigma/eps_r per element in sig (NULL = none)
@@ -110,7 +113,8 @@ hipError_t launch_stage(int order, const StageArgs<T>& a, int mode, int grid, hi
 template <typename T>
 int stage_blocks_per_cu(int order);
 
-int elements_per_block(int order);
+// small: StageArgs::small_blocks.
+int elements_per_block(int order, bool small = false);
 
 // Triangle (2D) stage kernel, dg_tri.hip: StageArgs with the triangle records
 // (geo: 15 values, conn: 6 ints per element; mats: Dr^T, Ds^T, LIFT^T; tabs:

@@ -13,17 +13,24 @@
 namespace dgtd {
 namespace valu {
 
-template <int P>
+// SMALL: element blocks half as large, for meshes that leave CUs idle
+// (StageArgs::small_blocks).  A block's LDS reads in the products go through
+// its CU's one LDS, so half the elements finish sooner: order 3 FP64, 48
+// tetrahedra: 8.3 -> 7.8 us per stage; order 1 FP32, 1,296: 5.2 -> 4.8; order 2
+// FP32, 3,072: 6.6 -> 6.0.  A quarter of the elements gains no more, and two
+// half blocks on a CU instead of one block lose (order 3 FP64, 3,072: 9.8 ->
+// 10.3 us).
+template <int P, bool SMALL = false>
 struct Shape {
     static constexpr int NP = (P + 1) * (P + 2) * (P + 3) / 6;
     static constexpr int NFP = (P + 1) * (P + 2) / 2;
     static constexpr int NF = 4 * NFP;
-    static constexpr int EB = (256 / NP) > 0 ? (256 / NP) : 1;  // elements per block
+    static constexpr int EB = (SMALL ? 128 : 256) / NP;  // elements per block
 };
 
-template <int P, typename T>
+template <int P, typename T, bool SMALL = false>
 struct Smem {
-    using S = Shape<P>;
+    using S = Shape<P, SMALL>;
     static constexpr int nD = 3 * S::NP * S::NP;
     static constexpr int nL = S::NF * S::NP;
     static constexpr int nQ = 6 * S::EB * S::NP;
@@ -38,9 +45,9 @@ struct Smem {
 constexpr int kThreads = 256;
 
 // A block's fields and records on their way from memory into LDS.
-template <int P, typename T>
+template <int P, typename T, bool SMALL = false>
 struct Fetched {
-    using S = Shape<P>;
+    using S = Shape<P, SMALL>;
     static constexpr int NG = (S::EB * kGeoStrideDev + kThreads - 1) / kThreads;
     static constexpr int NC = (S::EB * kConnStrideDev + kThreads - 1) / kThreads;
     T q[6], g[NG];
@@ -49,10 +56,10 @@ struct Fetched {
 
 // Issues every load of element block blk's fields and records (threads past
 // the end load a clamped, valid address).
-template <int P, typename T>
-__device__ __forceinline__ void stage_fetch(const StageArgs<T>& a, int blk, Fetched<P, T>& f)
+template <int P, typename T, bool SMALL = false>
+__device__ __forceinline__ void stage_fetch(const StageArgs<T>& a, int blk, Fetched<P, T, SMALL>& f)
 {
-    using S = Shape<P>;
+    using S = Shape<P, SMALL>;
     constexpr int NP = S::NP, EB = S::EB;
     const int tid = threadIdx.x;
     const size_t N = (size_t)NP * a.K;
@@ -64,12 +71,12 @@ __device__ __forceinline__ void stage_fetch(const StageArgs<T>& a, int blk, Fetc
 #pragma unroll
     for (int c = 0; c < 6; ++c) f.q[c] = a.qin[c * N + base + iq];
 #pragma unroll
-    for (int k = 0; k < Fetched<P, T>::NG; ++k) {
+    for (int k = 0; k < Fetched<P, T, SMALL>::NG; ++k) {
         const int i = tid + k * kThreads;
         f.g[k] = a.geo[(size_t)e0 * kGeoStrideDev + (i < ng ? i : ng - 1)];
     }
 #pragma unroll
-    for (int k = 0; k < Fetched<P, T>::NC; ++k) {
+    for (int k = 0; k < Fetched<P, T, SMALL>::NC; ++k) {
         const int i = tid + k * kThreads;
         f.c[k] = a.conn[(size_t)e0 * kConnStrideDev + (i < nc ? i : nc - 1)];
     }
@@ -79,12 +86,12 @@ __device__ __forceinline__ void stage_fetch(const StageArgs<T>& a, int blk, Fetc
 // stage_block's first barrier follows).  The tables' loads are issued before
 // the matrices', of which several are in flight per thread (up to 55 values
 // per thread at order 5), so one memory latency covers both.
-template <int P, typename T>
+template <int P, typename T, bool SMALL = false>
 __device__ __forceinline__ void stage_load_ref(const T* __restrict__ mats, const int* __restrict__ tabs,
                                                unsigned char* smem_raw)
 {
-    using S = Shape<P>;
-    using L = Smem<P, T>;
+    using S = Shape<P, SMALL>;
+    using L = Smem<P, T, SMALL>;
     constexpr int NT = 4 * S::NFP + 96 * S::NFP, NTT = (NT + kThreads - 1) / kThreads;
     T* sD = reinterpret_cast<T*>(smem_raw);
     int* sFm = reinterpret_cast<int*>(sD + L::nReal) + S::EB * kConnStrideDev;
@@ -108,12 +115,12 @@ __device__ __forceinline__ void stage_load_ref(const T* __restrict__ mats, const
 // GLOBAL: the Global operator's form of the same stage (GlobalEvolution.cpp:
 // 628-1088): SMA faces weighted as at alpha = 1 (DGOperatorFactory.h:485-495,
 // 587-591) and -sigma/eps E on the E rows (:1351-1361).
-template <int P, typename T, int MODE, bool GLOBAL = false, bool KEEP = false>
+template <int P, typename T, int MODE, bool GLOBAL = false, bool KEEP = false, bool SMALL = false>
 __device__ __forceinline__ void stage_block(const StageArgs<T>& a, unsigned char* smem_raw, int blk,
-                                            const Fetched<P, T>& fetched)
+                                            const Fetched<P, T, SMALL>& fetched)
 {
-    using S = Shape<P>;
-    using L = Smem<P, T>;
+    using S = Shape<P, SMALL>;
+    using L = Smem<P, T, SMALL>;
     constexpr int NP = S::NP, NFP = S::NFP, NF = S::NF, EB = S::EB;
     T* sD = reinterpret_cast<T*>(smem_raw);  // [3][j][i]
     T* sL = sD + L::nD;                      // [m][i]
@@ -138,10 +145,10 @@ __device__ __forceinline__ void stage_block(const StageArgs<T>& a, unsigned char
                 for (int c = 0; c < 6; ++c) sQ[c * EB * NP + tid] = fetched.q[c];
             }
 #pragma unroll
-            for (int k = 0; k < Fetched<P, T>::NG; ++k)
+            for (int k = 0; k < Fetched<P, T, SMALL>::NG; ++k)
                 if (tid + k * kThreads < ng) sG[tid + k * kThreads] = fetched.g[k];
 #pragma unroll
-            for (int k = 0; k < Fetched<P, T>::NC; ++k)
+            for (int k = 0; k < Fetched<P, T, SMALL>::NC; ++k)
                 if (tid + k * kThreads < nc) sC[tid + k * kThreads] = fetched.c[k];
         }
         __syncthreads();
