@@ -1,9 +1,8 @@
 // Stage kernel over the assembled Global operator (GlobalEvolution::Mult,
 // GlobalEvolution.cpp:628-1088, out = A [E; H]) in CSR: a block of 256
-// threads takes 256 / LPR rows (LPR lanes per row: 8 or 4 for the short rows of
-// hexahedra, the one shape that still runs it: on the others, and on
-// hexahedra unless the matrix is asked for, the operator is applied without
-// it), streams their entries (value, 16-bit column code, gathered state
+// threads takes 256 / LPR rows (LPR lanes per row: 16 for the long rows of
+// tetrahedra, 8 or 4 for the short rows of tensor-product elements and low
+// orders), streams their entries (value, 16-bit column code, gathered state
 // value) into LDS products, the LPR lanes of a row sum them, and the lane with
 // the sum applies the stage update of that DOF (rows are in the state layout).
 // HBM-bound on the matrix: per entry one value and a 16-bit element-local
@@ -71,14 +70,15 @@ __global__ __launch_bounds__(256) void csr_stage(StageArgs<T> a)
     const int64_t rb = a.rowptr[r], re = a.rowptr[r + 1];
     // The row's own stage operands do not depend on the product.  With short
     // rows and small chunks their loads are issued here and complete while the
-    // entries stream (measured: order-3 hexahedra FP32 571 -> 493 us); with
-    // larger chunks the two or four extra registers cost waves per SIMD and the
-    // loads stay after the product.
-    constexpr bool kEarly = kUnroll <= (sizeof(T) == 4 ? 5 : 4);
+    // entries stream (measured: order-3 quadrilaterals FP32 241 -> 219 us,
+    // FP64 304 -> 286 us; hexahedra FP32 571 -> 493 us); with larger chunks
+    // the two or four extra registers cost waves per SIMD and the loads stay
+    // after the product.
+    constexpr bool kEarly = LPR < 16 && kUnroll <= (sizeof(T) == 4 ? 5 : 4);
     T own0 = T(0), own1 = T(0);
     auto load_own = [&]() {
         if constexpr (MODE == kModeLserk) {
-            own0 = a.res_in ? a.res[r] : T(0);
+            own0 = a.res[r];
             own1 = a.qin[r];
         } else if constexpr (MODE == kModeRk1) {
             own0 = a.qin[r];
@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void csr_stage(StageArgs<T> a)
         a.out[r] = rhs;
     } else if constexpr (MODE == kModeLserk) {
         const T rr = a.ca * own0 + a.dt * rhs;
-        if (a.res_out) a.res[r] = rr;
+        a.res[r] = rr;
         const T qn = own1 + a.cb * rr;
         a.out[r] = qn;
         check(qn);
@@ -163,11 +163,16 @@ hipError_t csr_go(const StageArgs<T>& a, hipStream_t s)
 template <typename T, int MODE>
 hipError_t csr_launch(const StageArgs<T>& a, hipStream_t s)
 {
-    // Lanes per row by the average row length (18 entries on order-3
-    // hexahedra aligned with the axes, up to about 40 on sheared ones): a block
-    // takes 64 or 32 rows, so it still streams a full chunk.  One chunk per
-    // block where the rows allow: the smallest chunk holding an average
-    // block's entries, at most 1536 entries.
+    // Lanes per row by the average row length: short rows (13 entries on
+    // order-3 quadrilaterals and 18 on order-3 hexahedra aligned with the
+    // axes, 41 on order-1 hexahedra of a general shape) share a block among 64
+    // or 32 rows, so a block still streams a full chunk; long rows (50 / 57 /
+    // 63 / 70 on general hexahedra of orders 2-5, 156 on order-3 tetrahedra)
+    // take 16 lanes.  One chunk per block where the rows allow: the smallest
+    // chunk holding an average block's entries, at most 4096 entries.  General
+    // hexahedra with 8 lanes and two chunks of 1536 entries instead: order 4
+    // FP64 326 -> 348 us per stage at 1.6 million unknowns, 6.2 -> 7.6 us at
+    // 20,000; order 2 FP32 201 -> 210 and 7.4 -> 8.1 us.
     const double avg = (double)a.nnz / (double)a.nrows;
     if (avg <= 24.0) {
         const double per_block = avg * 64;
@@ -177,10 +182,19 @@ hipError_t csr_launch(const StageArgs<T>& a, hipStream_t s)
         if (per_block <= 256 * 5) return csr_go<T, MODE, 5, 4>(a, s);
         return csr_go<T, MODE, 6, 4>(a, s);
     }
-    const double per_block = avg * 32;
-    if (per_block <= 256 * 4) return csr_go<T, MODE, 4, 8>(a, s);
-    if (per_block <= 256 * 5) return csr_go<T, MODE, 5, 8>(a, s);
-    return csr_go<T, MODE, 6, 8>(a, s);
+    if (avg <= 48.0) {
+        const double per_block = avg * 32;
+        if (per_block <= 256 * 4) return csr_go<T, MODE, 4, 8>(a, s);
+        if (per_block <= 256 * 5) return csr_go<T, MODE, 5, 8>(a, s);
+        return csr_go<T, MODE, 6, 8>(a, s);
+    }
+    const double per_block = avg * 16;
+    if (per_block <= 256 * 5) return csr_go<T, MODE, 5, 16>(a, s);
+    if (per_block <= 256 * 8) return csr_go<T, MODE, 8, 16>(a, s);
+    if (sizeof(T) == 4 && per_block <= 256 * 10)  // FP64 measured faster with the 3072-entry chunk
+        return csr_go<T, MODE, 10, 16>(a, s);
+    if (per_block <= 256 * 12) return csr_go<T, MODE, 12, 16>(a, s);
+    return csr_go<T, MODE, 16, 16>(a, s);
 }
 
 }  // namespace

@@ -15,6 +15,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle_hex as OH
+from test_global_assembly import csr_matvec
 from test_oracle_hex import sheared_hexes
 
 pytestmark = pytest.mark.gpu
@@ -53,6 +54,32 @@ def test_hex_mult_matches_oracle(order):
         assert rel(g32.mult(x), yr) <= 1e-5
         g64.close()
         g32.close()
+
+
+@pytest.mark.parametrize("order", [2, 3, 4, 5])
+def test_hex_assembled_long_rows(order):
+    """Parallelepipeds of a general shape have more than 48 entries per row of
+    the assembled operator and take the stage's 16-lane rows: Mult and one
+    classic RK4 step (the matrix's Taylor polynomial) against the matrix."""
+    vx, E, bc = D.cartesian_3d(*(5, 5, 4) if order == 2 else (4, 3, 3), "hex")
+    vx = vx @ np.array([[1, 0.3, 0.2], [0.25, 0.9, 0.35], [0.15, 0.2, 1.1]]).T
+    sigma = np.random.default_rng(order).uniform(0, 3, E.shape[0])
+    A = D.global_assemble(vx, E, bc, order, sigma=sigma)
+    assert A[1].size > 48 * (A[0].size - 1)
+    x = np.random.default_rng(order).standard_normal(A[0].size - 1)
+    y = csr_matvec(A, x)
+    g64 = D.GlobalEvolution(vx, E, bc, order, sigma=sigma, precision=64, integrator="rk4")
+    assert np.abs(g64.mult(x) - y).max() <= 1e-12 * np.abs(y).max()
+    g32 = D.GlobalEvolution(vx, E, bc, order, sigma=sigma, precision=32)
+    assert rel(g32.mult(x), y) <= 1e-5
+    dt = 0.5 * np.linalg.norm(x) / np.linalg.norm(y)
+    z, k = x.copy(), x.copy()
+    for m in range(1, 5):
+        k = csr_matvec(A, k) * (dt / m)
+        z += k
+    g64.set_state(x)
+    g64.advance(dt, 1)
+    assert np.abs(g64.get_state() - z).max() <= 1e-12 * np.abs(z).max()
 
 
 def test_hex_kernel_choice_positions_and_probes():
