@@ -203,6 +203,7 @@ struct dgtd_op {
     int last_launches = 0;
 
     bool small_blocks = false;  // StageArgs::small_blocks
+    int cus = 1;                // compute units of the device (tensor-product stage)
     int64_t record_bytes = 0;  // geometry and connectivity records of the stage kernels
 
     // Below 12 MB per state buffer a stage runs from the L2s: the shortened
@@ -261,8 +262,8 @@ struct dgtd_op {
     hipError_t launch_on(const dgtd::StageArgs<T>& a0, int mode, int var, hipStream_t s) const
     {
         if (var == DGTD_KERNEL_CSR && !global_free) return dgtd::launch_csr_stage<T>(a0, mode, s);
-        if (hex) return dgtd::launch_tensor_stage<T>(H3.p, 3, a0, mode, s);
-        if (quad) return dgtd::launch_tensor_stage<T>(Q2.p, 2, a0, mode, s);
+        if (hex) return dgtd::launch_tensor_stage<T>(H3.p, 3, a0, mode, cus, s);
+        if (quad) return dgtd::launch_tensor_stage<T>(Q2.p, 2, a0, mode, cus, s);
         if (var == DGTD_KERNEL_MFMA) {
             dgtd::StageArgs<T> a = a0;
             a.mats = static_cast<const T*>(d_mats_mfma);
@@ -788,6 +789,7 @@ void upload_tensor(dgtd_op* op, int p, const std::vector<double>& host_geo, cons
                    const double* sigma, const std::vector<double>& eps, const std::vector<int>& fmask,
                    const std::vector<int>& perm)
 {
+    hip_check(hipDeviceGetAttribute(&op->cus, hipDeviceAttributeMultiprocessorCount, op->device), "compute units");
     const int K = op->K, n1 = p + 1, stride = (int)(host_geo.size() / K);
     std::vector<double> geo((size_t)(stride + 1) * K);
     for (int e = 0; e < K; ++e) {

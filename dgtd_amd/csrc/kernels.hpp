@@ -102,9 +102,9 @@ hipError_t launch_csr_stage(const StageArgs<T>& a, int mode, hipStream_t s);
 // Matrix-free stage of quadrilaterals (dim 2) and hexahedra (dim 3),
 // tensor_stage.hip: records as in tensor_dev.hpp, mats = D1 (row-major
 // (p+1)^2) then M1^-1 columns 0 and p ((p+1) x 2), tabs = Fmask [faces Nfp]
-// then the neighbour-node table (rows of Nfp).
+// then the neighbour-node table (rows of Nfp); cus: the device's compute units.
 template <typename T>
-hipError_t launch_tensor_stage(int order, int dim, const StageArgs<T>& a, int mode, hipStream_t s);
+hipError_t launch_tensor_stage(int order, int dim, const StageArgs<T>& a, int mode, int cus, hipStream_t s);
 
 template <typename T>
 hipError_t launch_stage(int order, const StageArgs<T>& a, int mode, int grid, hipStream_t s);

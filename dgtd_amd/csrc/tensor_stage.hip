@@ -8,27 +8,28 @@
 // costs 6 DIM (p+1) multiply-adds and the HBM traffic per DOF is the state
 // vectors and a share of the element's record.
 //
-// A block of six waves takes EB = 256 / Np elements:
-//   1. state (four values per access, whole lines) and records into LDS; the
-//      threads that form fluxes start their chain neighbour id -> neighbour
-//      node -> exterior trace at the same time;
+// A block takes EB = 256 / Np elements:
+//   1. state and records into LDS, a node per thread and its six components;
+//      the threads that form fluxes start their chain neighbour id ->
+//      neighbour node -> exterior trace before that;
 //   2. per face node: jump (or the boundary / interior-condition weights of
 //      the own trace), flux fluxE = a (dE - n (n . dE)) + n x dH, fluxH = a
 //      (dH - n (n . dH)) - n x dE, scaled by fscale/2 and 1/eps or 1/mu, into
-//      LDS; a = 1 on SMA faces whatever alpha, as the Global operator
-//      assembles them;
+//      LDS (component-major: component-last tiles, a stride of six words, made
+//      the banks collide); a = 1 on SMA faces whatever alpha, as the Global
+//      operator assembles them;
 //   3. per node: metric-weighted tensor derivatives of the six components,
-//      the curl, the lifted face fluxes, -sigma/eps E;
-//   4. the right-hand sides through LDS, then the stage update, four values
-//      per access.
-// What bounds it is the vector-memory address path, not HBM: a 4-byte access
-// of a wave occupies it as long as a 16-byte one, so state, records and update
-// move in wide accesses and only the traces are gathered value by value.
-// Measured per LSERK stage, order 3: 256^2 quadrilaterals FP64 46 us, FP32
-// 25 us (assembled matrix: 375 and 290 us on a mesh with no two elements
-// alike); 32^3 hexahedra FP64 141 us, FP32 55 us (164 and 57 us with 4-byte
-// accesses, records read from memory and component-last flux tiles, whose
-// stride of six words made the LDS banks collide).
+//      the curl, the lifted face fluxes, -sigma/eps E and the stage update of
+//      the node's six values.
+// Large meshes run at the memory rate, small ones at the latency of that chain.
+// An earlier form moved state and update in 16- and 32-byte accesses by six
+// waves, one component each; the right-hand sides then crossed LDS behind two
+// more barriers, a third of the waves idled in the products, and an FP64 lane's
+// 32 bytes half-filled each access.  Per stage, that form -> this one, 8
+// million unknowns: hexahedra order 1 FP64 106 -> 73 us (operator alone 97 ->
+// 63), order 3 FP32 38 -> 29 and FP64 75 -> 55, order 5 FP64 79 -> 57 (66 ->
+// 45); quadrilaterals order 3 FP32 29 -> 24 and FP64 54 -> 42, order 5 FP64
+// 65 -> 42.  Order-5 hexahedra in FP32 below 20,000 unknowns lose: 4.9 -> 5.0.
 #include <hip/hip_runtime.h>
 
 #include "kernels.hpp"
@@ -38,10 +39,6 @@
 namespace dgtd {
 
 namespace {
-
-// Six waves: one component's part of the block is at most 64 vectors of four
-// values, so each wave moves one component.
-constexpr int kThreads = 384;
 
 template <int P, int DIM>
 struct Tensor {
@@ -56,24 +53,15 @@ struct Tensor {
     static constexpr int METRIC = DIM * DIM;      // record: metric, faces (normal, fscale/2), 1/eps, 1/mu, sigma/eps
     static constexpr int FREC = DIM + 1;
     static constexpr int NE = EB * NP;            // values per component and block
-    static constexpr int FN = NF > NP ? NF : NP;  // LDS values per element and component: fluxes, then right-hand sides
 };
 
-// Four consecutive values, aligned to one value (the component stride is
-// arbitrary), which global accesses allow.
-template <typename T>
-struct Wide {
-    typedef T type __attribute__((ext_vector_type(4), aligned(sizeof(T))));
-};
-
-template <typename T, int P, int DIM, int MODE>
+template <typename T, int P, int DIM, int MODE, int kThreads>
 __global__ __launch_bounds__(kThreads) void tensor_stage(StageArgs<T> a)
 {
     using S = Tensor<P, DIM>;
-    constexpr int N1 = S::N1, NP = S::NP, NFP = S::NFP, NF = S::NF, EB = S::EB, NE = S::NE, FN = S::FN;
-    using v4 = typename Wide<T>::type;
+    constexpr int N1 = S::N1, NP = S::NP, NFP = S::NFP, NF = S::NF, EB = S::EB, NE = S::NE;
     __shared__ T sq[6 * NE];       // [c][el*NP + i]
-    __shared__ T sf[6 * EB * FN];  // fluxes [el][c][f*NFP + b], then right-hand sides [c][el*NP + i]
+    __shared__ T sf[6 * EB * NF];  // fluxes [el][c][f*NFP + b]
     __shared__ T sg[EB * S::GEO];
     __shared__ T sD[N1 * N1];
     __shared__ T sMi[N1 * 2];
@@ -86,47 +74,39 @@ __global__ __launch_bounds__(kThreads) void tensor_stage(StageArgs<T> a)
     const int e0 = blk * EB;
     if (e0 >= K) return;
     const int ne = min(EB, K - e0);
-    const bool full = ne == EB;
     const int cnt = ne * NP;
 
-    // ---- every load that depends on nothing ----
-    // lane l of wave c: values 4 l .. 4 l + 3 of component c's part of the
-    // block (lanes past the end repeat the last vector, which overlaps its
-    // predecessor when NE is no multiple of 4: the same values twice)
-    const int c0 = __builtin_amdgcn_readfirstlane(t / 64);
-    const int first = min(4 * (t % 64), NE - 4);
-    const size_t off = (size_t)c0 * N + (size_t)e0 * NP;
-    auto load = [&](const T* p) -> v4 {
-        v4 v;
-        if (full) {
-            v = *reinterpret_cast<const v4*>(p + off + first);
-        } else {
+    // ---- loads (threads past the end repeat the last node's or face node's) ----
+    // the longest chain first: neighbour and table row, neighbour node, trace
+    constexpr int NS = (EB * NF + kThreads - 1) / kThreads;
+    const int* fmask = a.tabs;      // [NFACE][NFP]
+    const int* perm = a.tabs + NF;  // neighbour-node table rows of NFP
+    int nb[NS], row[NS], own[NS];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = p[off + min(first + r, cnt - 1)];
-        }
-        return v;
-    };
-    const v4 q = load(a.qin);
+    for (int k = 0; k < NS; ++k) {
+        const int s = min(t + kThreads * k, ne * NF - 1);
+        const int el = s / NF, m = s - el * NF;
+        const size_t rec = (size_t)(e0 + el) * S::CONN + m / NFP;
+        nb[k] = a.conn[rec];
+        row[k] = a.conn[rec + S::NFACE];
+        own[k] = fmask[m];
+    }
+    const bool node = t < cnt;
+    const size_t own0 = (size_t)e0 * NP + min(t, cnt - 1);
+    T q[6];
+#pragma unroll
+    for (int c = 0; c < 6; ++c) q[c] = a.qin[c * N + own0];
     constexpr int NGL = (EB * S::GEO + kThreads - 1) / kThreads;
     T gv[NGL];
 #pragma unroll
     for (int k = 0; k < NGL; ++k) gv[k] = a.geo[(size_t)e0 * S::GEO + min(t + kThreads * k, ne * S::GEO - 1)];
-    // the thread's face nodes: neighbour, own and neighbour volume node
-    constexpr int NS = (EB * NF + kThreads - 1) / kThreads;
-    const int* fmask = a.tabs;      // [NFACE][NFP]
-    const int* perm = a.tabs + NF;  // neighbour-node table rows of NFP
-    int nb[NS], own[NS];
     T d[NS][6];
 #pragma unroll
     for (int k = 0; k < NS; ++k) {
         const int s = min(t + kThreads * k, ne * NF - 1);
-        const int el = s / NF, m = s - el * NF, f = m / NFP;
-        const size_t rec = (size_t)(e0 + el) * S::CONN;
-        nb[k] = a.conn[rec + f];
-        const int row = a.conn[rec + S::NFACE + f];
-        own[k] = fmask[m];
+        const int el = s / NF, m = s - el * NF;
         // a boundary face reads the element's own trace (replaced below)
-        const int pn = perm[(nb[k] >= 0 ? row : 0) * NFP + (m - f * NFP)];
+        const int pn = perm[(nb[k] >= 0 ? row[k] : 0) * NFP + m % NFP];
         const size_t g = nb[k] >= 0 ? (size_t)nb[k] * NP + pn : (size_t)(e0 + el) * NP + own[k];
 #pragma unroll
         for (int c = 0; c < 6; ++c) d[k][c] = a.qin[c * N + g];
@@ -134,15 +114,10 @@ __global__ __launch_bounds__(kThreads) void tensor_stage(StageArgs<T> a)
     // D1 row-major, then M1^-1 columns 0 and p
     if (t < N1 * N1) sD[t] = a.mats[t];
     if (t < N1 * 2) sMi[t] = a.mats[N1 * N1 + t];
-    // the update's operands, in flight until the end
-    constexpr bool kNeedRes = MODE != kModeMult && MODE != kModeRk1;
-    constexpr bool kNeedX = MODE == kModeRk2 || MODE == kModeRk3;
-    v4 rv = {T(0), T(0), T(0), T(0)}, xv;
-    if constexpr (kNeedRes)
-        if (MODE != kModeLserk || a.res_in) rv = load(a.res);
-    if constexpr (kNeedX) xv = load(a.x);
+    if (node) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) sq[c0 * NE + first + r] = q[r];
+        for (int c = 0; c < 6; ++c) sq[c * NE + t] = q[c];
+    }
 #pragma unroll
     for (int k = 0; k < NGL; ++k)
         if (t + kThreads * k < EB * S::GEO) sg[t + kThreads * k] = gv[k];
@@ -176,22 +151,33 @@ __global__ __launch_bounds__(kThreads) void tensor_stage(StageArgs<T> a)
         const T fs = fr[DIM];
         const T nE = n[0] * dk[0] + n[1] * dk[1] + n[2] * dk[2], nH = n[0] * dk[3] + n[1] * dk[4] + n[2] * dk[5];
         const T se = fs * g[S::GEO - 3], sh = fs * g[S::GEO - 2];
-        T* o = sf + el * 6 * FN + m;
+        T* o = sf + el * 6 * NF + m;
 #pragma unroll
         for (int x = 0; x < 3; ++x) {
             const int y = (x + 1) % 3, z = (x + 2) % 3;
-            o[x * FN] = se * (al * (dk[x] - n[x] * nE) + (n[y] * dk[3 + z] - n[z] * dk[3 + y]));
-            o[(3 + x) * FN] = sh * (al * (dk[3 + x] - n[x] * nH) - (n[y] * dk[z] - n[z] * dk[y]));
+            o[x * NF] = se * (al * (dk[x] - n[x] * nE) + (n[y] * dk[3 + z] - n[z] * dk[3 + y]));
+            o[(3 + x) * NF] = sh * (al * (dk[3 + x] - n[x] * nH) - (n[y] * dk[z] - n[z] * dk[y]));
         }
     }
     __syncthreads();
 
-    // ---- right-hand sides, a node per thread (the first NE threads) ----
-    const bool node = t < cnt;
+    // the update's operands, in flight during the products
+    constexpr bool kNeedRes = MODE == kModeLserk || MODE == kModeLserkLast || MODE == kModeRk2 || MODE == kModeRk3 ||
+                              MODE == kModeRk4;
+    constexpr bool kNeedX = MODE == kModeRk2 || MODE == kModeRk3;
+    T rv[6], xv[6];
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+        if constexpr (kNeedRes) rv[c] = a.res[c * N + own0];
+        if constexpr (kNeedX) xv[c] = a.x[c * N + own0];
+    }
+
+    // ---- right-hand sides and stage update, a node per thread (the first NE threads) ----
     const int el = t / NP, i = t - el * NP;
     const int ix = i % N1, iy = i / N1 % N1, iz = DIM == 3 ? i / NFP : 0;
-    T rhs[6];
+    bool bad = false;
     if (node) {
+        T rhs[6];
         const T* g = sg + el * S::GEO;
         const T* uo = sq + el * NP;
         // physical derivatives: D_d u = sum_k G[k][d] d_k u
@@ -226,9 +212,9 @@ __global__ __launch_bounds__(kThreads) void tensor_stage(StageArgs<T> a)
         // index][0 or p]
         auto lift = [&](int f, int line, int end, int b) {
             const T w = sMi[line * 2 + end];
-            const T* fl = sf + el * 6 * FN + f * NFP + b;
+            const T* fl = sf + el * 6 * NF + f * NFP + b;
 #pragma unroll
-            for (int c = 0; c < 6; ++c) rhs[c] += w * fl[c * FN];
+            for (int c = 0; c < 6; ++c) rhs[c] += w * fl[c * NF];
         };
         if constexpr (DIM == 3) {
             lift(0, iz, 0, ix + N1 * (P - iy));
@@ -243,94 +229,106 @@ __global__ __launch_bounds__(kThreads) void tensor_stage(StageArgs<T> a)
             lift(2, iy, 1, P - ix);
             lift(3, ix, 0, P - iy);
         }
-    }
-    __syncthreads();
-    if (node) {
 #pragma unroll
-        for (int c = 0; c < 6; ++c) sf[c * NE + t] = rhs[c];
-    }
-    __syncthreads();
-
-    // ---- stage update ----
-    bool bad = false;
-    v4 o, r2;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const T v = sf[c0 * NE + first + r], qv = q[r];
-        if constexpr (MODE == kModeMult) {
-            o[r] = v;
-        } else if constexpr (MODE == kModeLserk) {
-            r2[r] = a.ca * rv[r] + a.dt * v;
-            o[r] = qv + a.cb * r2[r];
-        } else if constexpr (MODE == kModeRk1) {
-            o[r] = qv + a.ca * v;
-            r2[r] = qv + a.cb * v;
-        } else if constexpr (MODE == kModeRk2 || MODE == kModeRk3) {
-            o[r] = xv[r] + a.ca * v;
-            r2[r] = rv[r] + a.cb * v;
-        } else {
-            o[r] = rv[r] + a.ca * v;
-        }
-        if constexpr (MODE == kModeLserk || MODE == kModeRk4) bad = bad || (first + r < cnt && unstable_entry(o[r]));
-    }
-    constexpr bool kRes = MODE != kModeMult && MODE != kModeRk4;
-    const bool keep = MODE != kModeLserk || a.res_out;
-    if (full) {
-        if constexpr (kRes)
-            if (keep) *reinterpret_cast<v4*>(a.res + off + first) = r2;
-        *reinterpret_cast<v4*>(a.out + off + first) = o;
-    } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (first + r < cnt) {
-                if constexpr (kRes)
-                    if (keep) a.res[off + first + r] = r2[r];
-                a.out[off + first + r] = o[r];
+        for (int c = 0; c < 6; ++c) {
+            const size_t o = c * N + own0;
+            if constexpr (MODE == kModeMult) {
+                a.out[o] = rhs[c];
+            } else if constexpr (is_lserk(MODE)) {
+                T r = a.dt * rhs[c];
+                if constexpr (MODE != kModeLserkFirst) r = a.ca * rv[c] + r;
+                const T qn = q[c] + a.cb * r;
+                if constexpr (MODE != kModeLserkLast) a.res[o] = r;
+                a.out[o] = qn;
+                bad = bad || unstable_entry(qn);
+            } else if constexpr (MODE == kModeRk1) {
+                a.out[o] = q[c] + a.ca * rhs[c];
+                a.res[o] = q[c] + a.cb * rhs[c];
+            } else if constexpr (MODE == kModeRk2 || MODE == kModeRk3) {
+                a.out[o] = xv[c] + a.ca * rhs[c];
+                a.res[o] = rv[c] + a.cb * rhs[c];
+            } else {
+                const T qn = rv[c] + a.ca * rhs[c];
+                a.out[o] = qn;
+                bad = bad || unstable_entry(qn);
             }
+        }
     }
-    if constexpr (MODE == kModeLserk || MODE == kModeRk4) report_unstable(a.unstable, bad);
+    if constexpr (is_lserk(MODE) || MODE == kModeRk4) report_unstable(a.unstable, bad);
+}
+
+template <typename T, int P, int DIM, int MODE, int kThreads>
+hipError_t tensor_threads(const StageArgs<T>& a, int blocks, hipStream_t s)
+{
+    hipLaunchKernelGGL((tensor_stage<T, P, DIM, MODE, kThreads>), dim3((unsigned)((blocks + 7) / 8 * 8)),
+                       dim3(kThreads), 0, s, a);
+    return hipGetLastError();
+}
+
+// Four waves, enough for a node per thread, or six where those form the
+// block's fluxes in one round fewer (hexahedra of orders 1, 3 and 4,
+// quadrilaterals of order 2) and the mesh is small: up to two blocks per CU
+// the round's latency counts (order 3 FP32, 1,331 hexahedra: 5.0 us with
+// four, 4.6 with six, the operator alone; order 4, 729: 5.7 and 5.2), beyond that
+// the idle waves of the products do (order 4, 10,648: 26.7 and 31.1).  Order
+// 1 in FP64 needs 58 KB of LDS, two blocks per CU, and takes six waves up to
+// one block per CU (10,648: 7.6 with four, 8.3 with six).  On order-2
+// quadrilaterals a third of the second round's threads have work and one round
+// stays ahead at every size (148,000, FP64: 38.2 with four, 35.9 with six).
+template <typename T, int P, int DIM, int MODE>
+hipError_t tensor_go(const StageArgs<T>& a, int cus, hipStream_t s)
+{
+    constexpr int EB = Tensor<P, DIM>::EB, F = EB * Tensor<P, DIM>::NF;
+    constexpr bool kSaves = (F + 383) / 384 < (F + 255) / 256;
+    const int blocks = (a.K + EB - 1) / EB;
+    if constexpr (kSaves && DIM == 2) {
+        return tensor_threads<T, P, DIM, MODE, 384>(a, blocks, s);
+    } else {
+        if constexpr (kSaves)
+            if (blocks <= (P == 1 && sizeof(T) == 8 ? 1 : 2) * cus)
+                return tensor_threads<T, P, DIM, MODE, 384>(a, blocks, s);
+        return tensor_threads<T, P, DIM, MODE, 256>(a, blocks, s);
+    }
 }
 
 template <typename T, int P, int DIM>
-hipError_t tensor_launch(const StageArgs<T>& a, int mode, hipStream_t s)
+hipError_t tensor_launch(const StageArgs<T>& a, int mode, int cus, hipStream_t s)
 {
-    constexpr int EB = Tensor<P, DIM>::EB;
-    const int blocks = (a.K + EB - 1) / EB;
-    const dim3 g((unsigned)((blocks + 7) / 8 * 8)), b(kThreads);
-    switch (mode) {
-        case kModeMult: hipLaunchKernelGGL((tensor_stage<T, P, DIM, kModeMult>), g, b, 0, s, a); break;
-        case kModeLserk: hipLaunchKernelGGL((tensor_stage<T, P, DIM, kModeLserk>), g, b, 0, s, a); break;
-        case kModeRk1: hipLaunchKernelGGL((tensor_stage<T, P, DIM, kModeRk1>), g, b, 0, s, a); break;
-        case kModeRk2: hipLaunchKernelGGL((tensor_stage<T, P, DIM, kModeRk2>), g, b, 0, s, a); break;
-        case kModeRk3: hipLaunchKernelGGL((tensor_stage<T, P, DIM, kModeRk3>), g, b, 0, s, a); break;
-        case kModeRk4: hipLaunchKernelGGL((tensor_stage<T, P, DIM, kModeRk4>), g, b, 0, s, a); break;
+    switch (lserk_mode(a, mode)) {
+        case kModeMult: return tensor_go<T, P, DIM, kModeMult>(a, cus, s);
+        case kModeLserk: return tensor_go<T, P, DIM, kModeLserk>(a, cus, s);
+        case kModeLserkFirst: return tensor_go<T, P, DIM, kModeLserkFirst>(a, cus, s);
+        case kModeLserkLast: return tensor_go<T, P, DIM, kModeLserkLast>(a, cus, s);
+        case kModeRk1: return tensor_go<T, P, DIM, kModeRk1>(a, cus, s);
+        case kModeRk2: return tensor_go<T, P, DIM, kModeRk2>(a, cus, s);
+        case kModeRk3: return tensor_go<T, P, DIM, kModeRk3>(a, cus, s);
+        case kModeRk4: return tensor_go<T, P, DIM, kModeRk4>(a, cus, s);
         default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 }  // namespace
 
 template <typename T>
-hipError_t launch_tensor_stage(int order, int dim, const StageArgs<T>& a, int mode, hipStream_t s)
+hipError_t launch_tensor_stage(int order, int dim, const StageArgs<T>& a, int mode, int cus, hipStream_t s)
 {
     if (a.K <= 0) return hipErrorInvalidValue;
     switch (10 * dim + order) {
-        case 21: return tensor_launch<T, 1, 2>(a, mode, s);
-        case 22: return tensor_launch<T, 2, 2>(a, mode, s);
-        case 23: return tensor_launch<T, 3, 2>(a, mode, s);
-        case 24: return tensor_launch<T, 4, 2>(a, mode, s);
-        case 25: return tensor_launch<T, 5, 2>(a, mode, s);
-        case 31: return tensor_launch<T, 1, 3>(a, mode, s);
-        case 32: return tensor_launch<T, 2, 3>(a, mode, s);
-        case 33: return tensor_launch<T, 3, 3>(a, mode, s);
-        case 34: return tensor_launch<T, 4, 3>(a, mode, s);
-        case 35: return tensor_launch<T, 5, 3>(a, mode, s);
+        case 21: return tensor_launch<T, 1, 2>(a, mode, cus, s);
+        case 22: return tensor_launch<T, 2, 2>(a, mode, cus, s);
+        case 23: return tensor_launch<T, 3, 2>(a, mode, cus, s);
+        case 24: return tensor_launch<T, 4, 2>(a, mode, cus, s);
+        case 25: return tensor_launch<T, 5, 2>(a, mode, cus, s);
+        case 31: return tensor_launch<T, 1, 3>(a, mode, cus, s);
+        case 32: return tensor_launch<T, 2, 3>(a, mode, cus, s);
+        case 33: return tensor_launch<T, 3, 3>(a, mode, cus, s);
+        case 34: return tensor_launch<T, 4, 3>(a, mode, cus, s);
+        case 35: return tensor_launch<T, 5, 3>(a, mode, cus, s);
         default: return hipErrorInvalidValue;
     }
 }
 
-template hipError_t launch_tensor_stage<float>(int, int, const StageArgs<float>&, int, hipStream_t);
-template hipError_t launch_tensor_stage<double>(int, int, const StageArgs<double>&, int, hipStream_t);
+template hipError_t launch_tensor_stage<float>(int, int, const StageArgs<float>&, int, int, hipStream_t);
+template hipError_t launch_tensor_stage<double>(int, int, const StageArgs<double>&, int, int, hipStream_t);
 
 }  // namespace dgtd

@@ -82,6 +82,33 @@ def test_hex_assembled_long_rows(order):
     assert np.abs(g64.get_state() - z).max() <= 1e-12 * np.abs(z).max()
 
 
+@pytest.mark.parametrize("order", [1, 3, 4])
+def test_hex_matrix_free_above_two_blocks_per_cu(order):
+    """Orders whose block has four waves above two blocks per compute unit and
+    six below: the first mesh above, with a partial last block, against the
+    assembled operator (Mult and two LSERK4 steps); the smaller meshes of the
+    other tests take six."""
+    block = 256 // (order + 1) ** 3
+    K = 2 * 256 * block + max(1, block - 1)  # 256 compute units
+    n = int(np.ceil(K ** (1 / 3)))
+    vx, E, bc = D.cartesian_3d(n, n, n, "hex", bc="sma")
+    vx = vx + 0.2 * vx[:, [1, 0, 2]]
+    E, bc = E[:K], bc[:K]
+    sigma = np.random.default_rng(order).uniform(0, 3, K)
+    kw = dict(sigma=sigma, alpha=0.5, precision=64)
+    free = D.HesthavenEvolution(vx, E, bc, order, kernel="valu", **kw)
+    full = D.GlobalEvolution(vx, E, bc, order, **kw)
+    x = np.random.default_rng(order).standard_normal(free.ndofs)
+    y = full.mult(x)
+    assert np.abs(free.mult(x) - y).max() <= 1e-12 * np.abs(y).max()
+    dt = 0.1 * np.linalg.norm(x) / np.linalg.norm(y)
+    for op in (free, full):
+        op.set_state(x)
+        op.advance(dt, 2)
+    z = full.get_state()
+    assert np.abs(free.get_state() - z).max() <= 1e-12 * np.abs(z).max()
+
+
 def test_hex_kernel_choice_positions_and_probes():
     vx, E, bc = sheared_hexes(2, 2, 1)
     op = D.HesthavenEvolution(vx, E, bc, 3)  # kernel "auto" takes the matrix-free hexahedron stage
