@@ -1,10 +1,11 @@
 // Stage kernel over the assembled Global operator (GlobalEvolution::Mult,
 // GlobalEvolution.cpp:628-1088, out = A [E; H]) in CSR: a block of 256
-// threads takes 256 / LPR rows (LPR lanes per row: 16 for the long rows of
-// tetrahedra, 8 or 4 for the short rows of tensor-product elements and low
-// orders), streams their entries (value, 16-bit column code, gathered state
+// threads takes 256 / LPR rows (LPR = 4, 8 or 16 lanes per row, by the rows'
+// length), streams their entries (value, 16-bit column code, gathered state
 // value) into LDS products, the LPR lanes of a row sum them, and the lane with
 // the sum applies the stage update of that DOF (rows are in the state layout).
+// Hexahedra run it when the matrix is asked for; the other shapes, and
+// hexahedra otherwise, apply the operator without it.
 // HBM-bound on the matrix: per entry one value and a 16-bit element-local
 // column code, decoded through the element table of the entry's 16-DOF group
 // (kCsrRowsPerBlock) in LDS.
@@ -163,13 +164,12 @@ hipError_t csr_go(const StageArgs<T>& a, hipStream_t s)
 template <typename T, int MODE>
 hipError_t csr_launch(const StageArgs<T>& a, hipStream_t s)
 {
-    // Lanes per row by the average row length: short rows (13 entries on
-    // order-3 quadrilaterals and 18 on order-3 hexahedra aligned with the
-    // axes, 41 on order-1 hexahedra of a general shape) share a block among 64
-    // or 32 rows, so a block still streams a full chunk; long rows (50 / 57 /
-    // 63 / 70 on general hexahedra of orders 2-5, 156 on order-3 tetrahedra)
-    // take 16 lanes.  One chunk per block where the rows allow: the smallest
-    // chunk holding an average block's entries, at most 4096 entries.  General
+    // Lanes per row by the average row length: short rows (18 entries on
+    // order-3 hexahedra aligned with the axes, 41 on order-1 hexahedra of a
+    // general shape) share a block among 64 or 32 rows, so a block still
+    // streams a full chunk; long rows (50 / 57 / 63 / 70 on general hexahedra
+    // of orders 2-5, at most 80) take 16 lanes.  One chunk per block where the
+    // rows allow: the smallest chunk holding an average block's entries.  General
     // hexahedra with 8 lanes and two chunks of 1536 entries instead: order 4
     // FP64 326 -> 348 us per stage at 1.6 million unknowns, 6.2 -> 7.6 us at
     // 20,000; order 2 FP32 201 -> 210 and 7.4 -> 8.1 us.
@@ -188,13 +188,7 @@ hipError_t csr_launch(const StageArgs<T>& a, hipStream_t s)
         if (per_block <= 256 * 5) return csr_go<T, MODE, 5, 8>(a, s);
         return csr_go<T, MODE, 6, 8>(a, s);
     }
-    const double per_block = avg * 16;
-    if (per_block <= 256 * 5) return csr_go<T, MODE, 5, 16>(a, s);
-    if (per_block <= 256 * 8) return csr_go<T, MODE, 8, 16>(a, s);
-    if (sizeof(T) == 4 && per_block <= 256 * 10)  // FP64 measured faster with the 3072-entry chunk
-        return csr_go<T, MODE, 10, 16>(a, s);
-    if (per_block <= 256 * 12) return csr_go<T, MODE, 12, 16>(a, s);
-    return csr_go<T, MODE, 16, 16>(a, s);
+    return csr_go<T, MODE, 5, 16>(a, s);
 }
 
 }  // namespace
