@@ -2,8 +2,8 @@
 
 #include <algorithm>
 #include <condition_variable>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -51,6 +51,7 @@ public:
     template <typename F>
     Workers(Progress& p, int count, int64_t blocks, F convert) : p_(p)
     {
+        threads_.reserve(count);
         for (int w = 0; w < count; ++w) {
             try {
                 threads_.emplace_back([&p, blocks, convert] {
@@ -68,8 +69,8 @@ public:
                         p.cv.notify_all();
                     }
                 });
-            } catch (const std::system_error&) {
-                break;  // no more threads: those that started do the work
+            } catch (const std::exception&) {
+                break;  // no more threads or memory for one: those that started do the work
             }
         }
     }
