@@ -1,8 +1,10 @@
 #include "host_copy.hpp"
 
 #include <algorithm>
+#include <array>
 #include <condition_variable>
 #include <exception>
+#include <memory>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -20,6 +22,112 @@ constexpr int64_t kDirectBytes = int64_t(8) << 20;
 constexpr int64_t kThreadBytes = int64_t(32) << 20;
 constexpr int64_t kBytesPerWorker = int64_t(4) << 20;
 constexpr int kMaxWorkers = 8;
+
+constexpr int kBlocks = 12;
+constexpr size_t kBytes = size_t(1) << 20;
+constexpr size_t kIdleRings = 2;
+
+// Pinned blocks and the events that say when the copy engine is done with them.
+struct Ring {
+    int device = 0;
+    void* block[kBlocks] = {};
+    hipEvent_t event[kBlocks] = {};
+
+    explicit Ring(int dev) : device(dev) {}
+    Ring(const Ring&) = delete;
+    Ring& operator=(const Ring&) = delete;
+    ~Ring()
+    {
+        for (int b = 0; b < kBlocks; ++b) {
+            if (block[b]) (void)hipHostFree(block[b]);
+            if (event[b]) (void)hipEventDestroy(event[b]);
+        }
+    }
+    hipError_t prepare()
+    {
+        for (int b = 0; b < kBlocks; ++b) {
+            if (!block[b])
+                if (const hipError_t e = hipHostMalloc(&block[b], kBytes, hipHostMallocDefault); e != hipSuccess) {
+                    block[b] = nullptr;
+                    return e;
+                }
+            if (!event[b])
+                if (const hipError_t e = hipEventCreateWithFlags(&event[b], hipEventDisableTiming); e != hipSuccess) {
+                    event[b] = nullptr;
+                    return e;
+                }
+        }
+        return hipSuccess;
+    }
+};
+
+// The process's idle rings: at most kIdleRings, freed with the last HostCopy.
+// A transfer borrows one for its duration, so transfers of any threads, on one
+// operator too, never share blocks.
+class Rings {
+public:
+    static Rings& get()
+    {
+        static Rings* r = new Rings;  // outlives every HostCopy
+        return *r;
+    }
+    void add_owner()
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        ++owners_;
+    }
+    void drop_owner()
+    {
+        std::array<std::unique_ptr<Ring>, kIdleRings> last;
+        std::lock_guard<std::mutex> lk(mu_);
+        if (--owners_ == 0) last.swap(idle_);
+    }
+    std::unique_ptr<Ring> take()
+    {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            for (auto& r : idle_)
+                if (r && r->device == dev) return std::move(r);
+        }
+        return std::make_unique<Ring>(dev);
+    }
+    void give(std::unique_ptr<Ring> r)
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        for (auto& slot : idle_)
+            if (!slot) {
+                slot = std::move(r);
+                return;
+            }
+    }
+
+private:
+    std::mutex mu_;
+    std::array<std::unique_ptr<Ring>, kIdleRings> idle_;
+    int owners_ = 0;
+};
+
+// A ring for one transfer, with its blocks (NULL: no pinned memory left).
+class Borrowed {
+public:
+    Borrowed() : ring_(Rings::get().take())
+    {
+        if (ring_ && ring_->prepare() != hipSuccess) {
+            (void)hipGetLastError();
+            ring_.reset();
+        }
+    }
+    ~Borrowed()
+    {
+        if (ring_) Rings::get().give(std::move(ring_));
+    }
+    Ring* get() const { return ring_.get(); }
+
+private:
+    std::unique_ptr<Ring> ring_;
+};
 
 // Progress of the blocks of one transfer, passed between the calling thread
 // (which drives the copy engine) and the workers (which convert).
@@ -126,51 +234,26 @@ hipError_t direct_to_device(const double* h, T* d, int64_t n, hipStream_t s)
 
 }  // namespace
 
-hipError_t HostCopy::prepare()
-{
-    if (ready_) return hipSuccess;
-    for (int b = 0; b < kBlocks; ++b) {
-        if (!block_[b])
-            if (const hipError_t e = hipHostMalloc(&block_[b], kBytes, hipHostMallocDefault); e != hipSuccess) {
-                block_[b] = nullptr;
-                return e;
-            }
-        if (!event_[b])
-            if (const hipError_t e = hipEventCreateWithFlags(&event_[b], hipEventDisableTiming); e != hipSuccess) {
-                event_[b] = nullptr;
-                return e;
-            }
-    }
-    ready_ = true;
-    return hipSuccess;
-}
-
-HostCopy::~HostCopy()
-{
-    for (int b = 0; b < kBlocks; ++b) {
-        if (block_[b]) (void)hipHostFree(block_[b]);
-        if (event_[b]) (void)hipEventDestroy(event_[b]);
-    }
-}
+HostCopy::HostCopy() { Rings::get().add_owner(); }
+HostCopy::~HostCopy() { Rings::get().drop_owner(); }
 
 template <typename T>
 hipError_t HostCopy::to_host(const T* d, double* h, int64_t n, hipStream_t s)
 {
     const int64_t bytes = n * (int64_t)sizeof(double);
     if (bytes < kDirectBytes) return direct_to_host(d, h, n, s);
-    if (prepare() != hipSuccess) {  // no pinned memory left
-        (void)hipGetLastError();
-        return direct_to_host(d, h, n, s);
-    }
+    const Borrowed borrowed;
+    Ring* const ring = borrowed.get();
+    if (!ring) return direct_to_host(d, h, n, s);
     const int64_t per = (int64_t)(kBytes / sizeof(T)), blocks = (n + per - 1) / per;
     auto copy = [&](int64_t i) {
         const int b = (int)(i % kBlocks);
-        hipError_t e = hipMemcpyAsync(block_[b], d + i * per, sizeof(T) * std::min(per, n - i * per),
+        hipError_t e = hipMemcpyAsync(ring->block[b], d + i * per, sizeof(T) * std::min(per, n - i * per),
                                       hipMemcpyDeviceToHost, s);
-        return e != hipSuccess ? e : hipEventRecord(event_[b], s);
+        return e != hipSuccess ? e : hipEventRecord(ring->event[b], s);
     };
-    auto convert = [=, this](int64_t i) {
-        const T* src = static_cast<const T*>(block_[i % kBlocks]);
+    auto convert = [=](int64_t i) {
+        const T* src = static_cast<const T*>(ring->block[i % kBlocks]);
         std::copy(src, src + std::min(per, n - i * per), h + i * per);
     };
     // copies run ahead of the conversions by the ring's length
@@ -179,7 +262,7 @@ hipError_t HostCopy::to_host(const T* d, double* h, int64_t n, hipStream_t s)
     if (bytes < kThreadBytes) {
         for (int64_t i = 0; i < blocks && e == hipSuccess; ++i) {
             while (e == hipSuccess && issued < std::min<int64_t>(blocks, i + kBlocks)) e = copy(issued++);
-            if (e == hipSuccess) e = hipEventSynchronize(event_[i % kBlocks]);
+            if (e == hipSuccess) e = hipEventSynchronize(ring->event[i % kBlocks]);
             if (e == hipSuccess) convert(i);
         }
         if (e != hipSuccess) (void)hipStreamSynchronize(s);
@@ -199,7 +282,7 @@ hipError_t HostCopy::to_host(const T* d, double* h, int64_t n, hipStream_t s)
             e = copy(issued);
             if (e == hipSuccess) ++issued;
         }
-        if (e == hipSuccess) e = hipEventSynchronize(event_[i % kBlocks]);
+        if (e == hipSuccess) e = hipEventSynchronize(ring->event[i % kBlocks]);
         if (e == hipSuccess) p.set_open(i + 1);
     }
     for (int64_t i = std::max<int64_t>(0, blocks - kBlocks); i < blocks && e == hipSuccess; ++i) p.wait_converted(i);
@@ -212,25 +295,24 @@ hipError_t HostCopy::to_device(const double* h, T* d, int64_t n, hipStream_t s)
 {
     const int64_t bytes = n * (int64_t)sizeof(double);
     if (bytes < kDirectBytes) return direct_to_device(h, d, n, s);
-    if (prepare() != hipSuccess) {
-        (void)hipGetLastError();
-        return direct_to_device(h, d, n, s);
-    }
+    const Borrowed borrowed;
+    Ring* const ring = borrowed.get();
+    if (!ring) return direct_to_device(h, d, n, s);
     const int64_t per = (int64_t)(kBytes / sizeof(T)), blocks = (n + per - 1) / per;
     auto copy = [&](int64_t i) {
         const int b = (int)(i % kBlocks);
-        hipError_t e = hipMemcpyAsync(d + i * per, block_[b], sizeof(T) * std::min(per, n - i * per),
+        hipError_t e = hipMemcpyAsync(d + i * per, ring->block[b], sizeof(T) * std::min(per, n - i * per),
                                       hipMemcpyHostToDevice, s);
-        return e != hipSuccess ? e : hipEventRecord(event_[b], s);
+        return e != hipSuccess ? e : hipEventRecord(ring->event[b], s);
     };
-    auto convert = [=, this](int64_t i) {
+    auto convert = [=](int64_t i) {
         const double* src = h + i * per;
-        std::copy(src, src + std::min(per, n - i * per), static_cast<T*>(block_[i % kBlocks]));
+        std::copy(src, src + std::min(per, n - i * per), static_cast<T*>(ring->block[i % kBlocks]));
     };
     hipError_t e = hipSuccess;
     if (bytes < kThreadBytes) {
         for (int64_t i = 0; i < blocks && e == hipSuccess; ++i) {
-            if (i >= kBlocks) e = hipEventSynchronize(event_[i % kBlocks]);
+            if (i >= kBlocks) e = hipEventSynchronize(ring->event[i % kBlocks]);
             if (e != hipSuccess) break;
             convert(i);
             e = copy(i);
@@ -249,7 +331,7 @@ hipError_t HostCopy::to_device(const double* h, T* d, int64_t n, hipStream_t s)
         // half a ring behind, the block is free again
         const int64_t done = i - kBlocks / 2;
         if (e == hipSuccess && done >= 0) {
-            e = hipEventSynchronize(event_[done % kBlocks]);
+            e = hipEventSynchronize(ring->event[done % kBlocks]);
             if (e == hipSuccess) p.set_open(std::min<int64_t>(blocks, done + 1 + kBlocks));
         }
     }

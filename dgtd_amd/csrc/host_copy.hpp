@@ -17,11 +17,12 @@
 
 namespace dgtd {
 
-// One owner's ring; calls on it are serialised by the owner.  The pinned
-// blocks are allocated by the first large transfer and freed with the owner.
+// The transfers of one operator or batch, from any threads.  Each borrows a
+// ring of pinned blocks; the process keeps at most two idle ones and frees them
+// with the last HostCopy.
 class HostCopy {
 public:
-    HostCopy() = default;
+    HostCopy();
     HostCopy(const HostCopy&) = delete;
     HostCopy& operator=(const HostCopy&) = delete;
     ~HostCopy();
@@ -32,14 +33,6 @@ public:
     // d[i] = h[i] on s; h stays valid until s has drained.
     template <typename T>
     hipError_t to_device(const double* h, T* d, int64_t n, hipStream_t s);
-
-private:
-    static constexpr int kBlocks = 12;
-    static constexpr size_t kBytes = size_t(1) << 20;
-    void* block_[kBlocks] = {};
-    hipEvent_t event_[kBlocks] = {};
-    bool ready_ = false;
-    hipError_t prepare();
 };
 
 }  // namespace dgtd

@@ -312,6 +312,30 @@ void no_pinned_memory()
         }
 }
 
+// Transfers of several threads, through one object and through several: no
+// block is shared, and at most 24 MB stay pinned between them.
+void threads()
+{
+    std::vector<dgtd::HostCopy> c(3);
+    for (const bool one : {true, false}) {
+        std::vector<std::thread> th;
+        for (int t = 0; t < 3; ++t)
+            th.emplace_back([&, t] {
+                for (int64_t n : {int64_t(2500001), int64_t(5000003)}) {
+                    const auto d = device_values<float>(n, 10 + t);
+                    std::vector<double> h(n, -1.0);
+                    check(c[one ? 0 : t].to_host(d.data(), h.data(), n, nullptr) == hipSuccess && same(d, h),
+                          "to_host of one of three threads");
+                    std::vector<float> back(n);
+                    check(c[one ? 0 : t].to_device(h.data(), back.data(), n, nullptr) == hipSuccess && back == d,
+                          "to_device of one of three threads");
+                }
+            });
+        for (auto& t : th) t.join();
+        check(g_pinned <= 24 << 20, "pinned memory kept");
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -321,6 +345,7 @@ int main(int argc, char** argv)
         {"failing_allocations", failing_allocations},
         {"failing_copies", failing_copies},
         {"no_pinned_memory", no_pinned_memory},
+        {"threads", threads},
     };
     const auto t = argc > 1 ? tests.find(argv[1]) : tests.end();
     if (t == tests.end()) return 2;
