@@ -23,29 +23,40 @@ constexpr int64_t kThreadBytes = int64_t(32) << 20;
 constexpr int64_t kBytesPerWorker = int64_t(4) << 20;
 constexpr int kMaxWorkers = 8;
 
-constexpr int kBlocks = 12;
+constexpr int kMaxBlocks = 12;
 constexpr size_t kBytes = size_t(1) << 20;
 constexpr size_t kIdleRings = 2;
+
+// Blocks of the ring a transfer uses, and so pins if nobody did before (85 us
+// each, and up to 370 us at its first touch): two suffice while the calling
+// thread converts (9 MB of FP32 unknowns, first and next download: 259 and 193
+// us with two, 587 and 183 with twelve, 440 directly; the first in a process
+// took 2-5 ms with twelve), eight and more keep the workers busy (38 MB: 1.7
+// ms with eight or twelve, 2.1-2.8 with six or four).
+int ring_blocks(int64_t host_bytes)
+{
+    return host_bytes < kThreadBytes ? 2 : (int)std::min<int64_t>(kMaxBlocks, host_bytes / (int64_t(4) << 20));
+}
 
 // Pinned blocks and the events that say when the copy engine is done with them.
 struct Ring {
     int device = 0;
-    void* block[kBlocks] = {};
-    hipEvent_t event[kBlocks] = {};
+    void* block[kMaxBlocks] = {};
+    hipEvent_t event[kMaxBlocks] = {};
 
     explicit Ring(int dev) : device(dev) {}
     Ring(const Ring&) = delete;
     Ring& operator=(const Ring&) = delete;
     ~Ring()
     {
-        for (int b = 0; b < kBlocks; ++b) {
+        for (int b = 0; b < kMaxBlocks; ++b) {
             if (block[b]) (void)hipHostFree(block[b]);
             if (event[b]) (void)hipEventDestroy(event[b]);
         }
     }
-    hipError_t prepare()
+    hipError_t prepare(int blocks)
     {
-        for (int b = 0; b < kBlocks; ++b) {
+        for (int b = 0; b < blocks; ++b) {
             if (!block[b])
                 if (const hipError_t e = hipHostMalloc(&block[b], kBytes, hipHostMallocDefault); e != hipSuccess) {
                     block[b] = nullptr;
@@ -109,12 +120,12 @@ private:
     int owners_ = 0;
 };
 
-// A ring for one transfer, with its blocks (NULL: no pinned memory left).
+// A ring for one transfer, with that many blocks (NULL: no pinned memory left).
 class Borrowed {
 public:
-    Borrowed() : ring_(Rings::get().take())
+    explicit Borrowed(int blocks) : ring_(Rings::get().take())
     {
-        if (ring_ && ring_->prepare() != hipSuccess) {
+        if (ring_ && ring_->prepare(blocks) != hipSuccess) {
             (void)hipGetLastError();
             ring_.reset();
         }
@@ -242,18 +253,19 @@ hipError_t HostCopy::to_host(const T* d, double* h, int64_t n, hipStream_t s)
 {
     const int64_t bytes = n * (int64_t)sizeof(double);
     if (bytes < kDirectBytes) return direct_to_host(d, h, n, s);
-    const Borrowed borrowed;
+    const int nring = ring_blocks(bytes);
+    const Borrowed borrowed(nring);
     Ring* const ring = borrowed.get();
     if (!ring) return direct_to_host(d, h, n, s);
     const int64_t per = (int64_t)(kBytes / sizeof(T)), blocks = (n + per - 1) / per;
     auto copy = [&](int64_t i) {
-        const int b = (int)(i % kBlocks);
+        const int b = (int)(i % nring);
         hipError_t e = hipMemcpyAsync(ring->block[b], d + i * per, sizeof(T) * std::min(per, n - i * per),
                                       hipMemcpyDeviceToHost, s);
         return e != hipSuccess ? e : hipEventRecord(ring->event[b], s);
     };
     auto convert = [=](int64_t i) {
-        const T* src = static_cast<const T*>(ring->block[i % kBlocks]);
+        const T* src = static_cast<const T*>(ring->block[i % nring]);
         std::copy(src, src + std::min(per, n - i * per), h + i * per);
     };
     // copies run ahead of the conversions by the ring's length
@@ -261,8 +273,8 @@ hipError_t HostCopy::to_host(const T* d, double* h, int64_t n, hipStream_t s)
     int64_t issued = 0;
     if (bytes < kThreadBytes) {
         for (int64_t i = 0; i < blocks && e == hipSuccess; ++i) {
-            while (e == hipSuccess && issued < std::min<int64_t>(blocks, i + kBlocks)) e = copy(issued++);
-            if (e == hipSuccess) e = hipEventSynchronize(ring->event[i % kBlocks]);
+            while (e == hipSuccess && issued < std::min<int64_t>(blocks, i + nring)) e = copy(issued++);
+            if (e == hipSuccess) e = hipEventSynchronize(ring->event[i % nring]);
             if (e == hipSuccess) convert(i);
         }
         if (e != hipSuccess) (void)hipStreamSynchronize(s);
@@ -273,19 +285,19 @@ hipError_t HostCopy::to_host(const T* d, double* h, int64_t n, hipStream_t s)
     Workers workers(p, worker_count(bytes), blocks, convert);
     if (workers.empty()) return direct_to_host(d, h, n, s);
     for (int64_t i = 0; i < blocks && e == hipSuccess; ++i) {
-        while (e == hipSuccess && issued < blocks && issued < i + kBlocks) {
-            if (issued >= kBlocks) {
+        while (e == hipSuccess && issued < blocks && issued < i + nring) {
+            if (issued >= nring) {
                 std::unique_lock<std::mutex> lk(p.mu);
-                if (!p.converted[issued - kBlocks] && issued > i) break;  // refill later
-                p.cv.wait(lk, [&] { return p.converted[issued - kBlocks] != 0; });
+                if (!p.converted[issued - nring] && issued > i) break;  // refill later
+                p.cv.wait(lk, [&] { return p.converted[issued - nring] != 0; });
             }
             e = copy(issued);
             if (e == hipSuccess) ++issued;
         }
-        if (e == hipSuccess) e = hipEventSynchronize(ring->event[i % kBlocks]);
+        if (e == hipSuccess) e = hipEventSynchronize(ring->event[i % nring]);
         if (e == hipSuccess) p.set_open(i + 1);
     }
-    for (int64_t i = std::max<int64_t>(0, blocks - kBlocks); i < blocks && e == hipSuccess; ++i) p.wait_converted(i);
+    for (int64_t i = std::max<int64_t>(0, blocks - nring); i < blocks && e == hipSuccess; ++i) p.wait_converted(i);
     if (e != hipSuccess) (void)hipStreamSynchronize(s);  // no copy into the ring outlives the call
     return e;
 }
@@ -293,26 +305,29 @@ hipError_t HostCopy::to_host(const T* d, double* h, int64_t n, hipStream_t s)
 template <typename T>
 hipError_t HostCopy::to_device(const double* h, T* d, int64_t n, hipStream_t s)
 {
+    // FP64: nothing to convert, and the source's pages exist (a plain copy of 10-250
+    // MB is as fast or up to a third faster than the ring)
     const int64_t bytes = n * (int64_t)sizeof(double);
-    if (bytes < kDirectBytes) return direct_to_device(h, d, n, s);
-    const Borrowed borrowed;
+    if (bytes < kDirectBytes || sizeof(T) == sizeof(double)) return direct_to_device(h, d, n, s);
+    const int nring = ring_blocks(bytes);
+    const Borrowed borrowed(nring);
     Ring* const ring = borrowed.get();
     if (!ring) return direct_to_device(h, d, n, s);
     const int64_t per = (int64_t)(kBytes / sizeof(T)), blocks = (n + per - 1) / per;
     auto copy = [&](int64_t i) {
-        const int b = (int)(i % kBlocks);
+        const int b = (int)(i % nring);
         hipError_t e = hipMemcpyAsync(d + i * per, ring->block[b], sizeof(T) * std::min(per, n - i * per),
                                       hipMemcpyHostToDevice, s);
         return e != hipSuccess ? e : hipEventRecord(ring->event[b], s);
     };
     auto convert = [=](int64_t i) {
         const double* src = h + i * per;
-        std::copy(src, src + std::min(per, n - i * per), static_cast<T*>(ring->block[i % kBlocks]));
+        std::copy(src, src + std::min(per, n - i * per), static_cast<T*>(ring->block[i % nring]));
     };
     hipError_t e = hipSuccess;
     if (bytes < kThreadBytes) {
         for (int64_t i = 0; i < blocks && e == hipSuccess; ++i) {
-            if (i >= kBlocks) e = hipEventSynchronize(ring->event[i % kBlocks]);
+            if (i >= nring) e = hipEventSynchronize(ring->event[i % nring]);
             if (e != hipSuccess) break;
             convert(i);
             e = copy(i);
@@ -322,17 +337,17 @@ hipError_t HostCopy::to_device(const double* h, T* d, int64_t n, hipStream_t s)
     }
     Progress p;
     p.converted.assign(blocks, 0);
-    p.open = std::min<int64_t>(blocks, kBlocks);
+    p.open = std::min<int64_t>(blocks, nring);
     Workers workers(p, worker_count(bytes), blocks, convert);
     if (workers.empty()) return direct_to_device(h, d, n, s);
     for (int64_t i = 0; i < blocks && e == hipSuccess; ++i) {
         p.wait_converted(i);
         e = copy(i);
         // half a ring behind, the block is free again
-        const int64_t done = i - kBlocks / 2;
+        const int64_t done = i - nring / 2;
         if (e == hipSuccess && done >= 0) {
-            e = hipEventSynchronize(ring->event[done % kBlocks]);
-            if (e == hipSuccess) p.set_open(std::min<int64_t>(blocks, done + 1 + kBlocks));
+            e = hipEventSynchronize(ring->event[done % nring]);
+            if (e == hipSuccess) p.set_open(std::min<int64_t>(blocks, done + 1 + nring));
         }
     }
     const hipError_t w = hipStreamSynchronize(s);

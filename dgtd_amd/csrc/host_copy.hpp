@@ -7,7 +7,8 @@
 // host vector and one more pass by the calling thread, and the first touch of
 // a fresh destination, page by page, stays on that thread too.  Measured for
 // 41.3 million FP32 unknowns (165 MB on the device, 330 MB on the host):
-// download 59 ms -> 6.1 ms, upload 38 -> 5.7 ms (FP64: 32 -> 11 and 11 -> 11).
+// download 59 ms -> 6.1 ms, upload 38 -> 5.7 ms (FP64 download 32 -> 11 ms; FP64
+// uploads, which convert nothing, stay plain copies).
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -336,6 +336,29 @@ void threads()
     }
 }
 
+// What a transfer pins: nothing below 8 MB or for an FP64 upload, 2 MB below
+// 32 MB, at most 12 MB.
+void pinned_memory()
+{
+    auto pins = [](int64_t n, auto value, bool up) {
+        using T = decltype(value);
+        std::vector<T> d(n);
+        std::vector<double> h(n);
+        dgtd::HostCopy c;
+        check((up ? c.to_device(h.data(), d.data(), n, nullptr) : c.to_host(d.data(), h.data(), n, nullptr)) == hipSuccess,
+              "transfer");
+        (void)hipStreamSynchronize(nullptr);
+        return (int64_t)g_pinned;
+    };
+    check(pins(1000000, 0.0f, false) == 0 && pins(1000000, 0.0, true) == 0, "nothing below 8 MB");
+    check(pins(1500000, 0.0, true) == 0 && pins(9000001, 0.0, true) == 0, "nothing for an FP64 upload");
+    for (const bool up : {false, true}) {
+        check(pins(1500000, 0.0f, up) <= 2 << 20 && pins(4000000, 0.0f, up) <= 2 << 20, "2 MB below 32 MB");
+        check(pins(9000001, 0.0f, up) <= 12 << 20 && pins(20000000, 0.0f, up) <= 12 << 20, "12 MB");
+    }
+    check(pins(4000000, 0.0, false) <= 2 << 20, "2 MB below 32 MB, FP64");
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -346,6 +369,7 @@ int main(int argc, char** argv)
         {"failing_copies", failing_copies},
         {"no_pinned_memory", no_pinned_memory},
         {"threads", threads},
+        {"pinned_memory", pinned_memory},
     };
     const auto t = argc > 1 ? tests.find(argv[1]) : tests.end();
     if (t == tests.end()) return 2;

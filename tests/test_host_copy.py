@@ -18,7 +18,8 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("test", ["round_trips", "failing_allocations", "failing_copies", "no_pinned_memory", "threads"])
+@pytest.mark.parametrize("test", ["round_trips", "failing_allocations", "failing_copies", "no_pinned_memory", "threads",
+                                  "pinned_memory"])
 def test_host_copy(program, test):
     r = subprocess.run([program, test], capture_output=True, text=True, timeout=120)
     print(r.stdout, r.stderr)
