@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <limits>
 #include <map>
 #include <mutex>
 #include <new>
@@ -75,13 +76,12 @@ void* upload(const std::vector<T>& h)
 
 namespace {
 // Process-wide autotuning cache: the chosen candidate per (element shape,
-// order, precision, stage mode, size class = floor(log2 K)).
+// order, precision, stage mode, size class = floor(log2 K), form of the stage
+// kernels: dgtd_op::tune_form, whose bounds lie inside a size class).
 struct TuneKey {
-    int dim, order, precision, mode, size_class;
-    bool operator<(const TuneKey& o) const
-    {
-        return std::tie(dim, order, precision, mode, size_class) < std::tie(o.dim, o.order, o.precision, o.mode, o.size_class);
-    }
+    int dim, order, precision, mode, size_class, form;
+    auto fields() const { return std::tie(dim, order, precision, mode, size_class, form); }
+    bool operator<(const TuneKey& o) const { return fields() < o.fields(); }
 };
 // The fastest candidate overall, the fastest matrix-core candidate (-1:
 // none) and every candidate's time in microseconds (0: did not fit).
@@ -102,19 +102,33 @@ int size_class(int64_t K)
     return c;
 }
 
-bool tune_cache_get(int dim, int order, int precision, int mode, int64_t K, TuneChoice& choice)
+bool tune_cache_get(int dim, int order, int precision, int mode, int64_t K, int form, TuneChoice& choice)
 {
     std::lock_guard<std::mutex> lk(g_tune_mu);
-    const auto it = g_tune.find(TuneKey{dim, order, precision, mode, size_class(K)});
+    const auto it = g_tune.find(TuneKey{dim, order, precision, mode, size_class(K), form});
     if (it == g_tune.end()) return false;
     choice = it->second;
     return true;
 }
 
-void tune_cache_put(int dim, int order, int precision, int mode, int64_t K, TuneChoice choice)
+// The choice made for any form of the stage kernels.
+bool tune_cache_get_any(int dim, int order, int precision, int mode, int64_t K, TuneChoice& choice)
 {
     std::lock_guard<std::mutex> lk(g_tune_mu);
-    g_tune[TuneKey{dim, order, precision, mode, size_class(K)}] = choice;
+    const TuneKey first{dim, order, precision, mode, size_class(K), std::numeric_limits<int>::min()};
+    const auto it = g_tune.lower_bound(first);
+    if (it == g_tune.end()) return false;
+    TuneKey found = it->first;
+    found.form = first.form;
+    if (first < found || found < first) return false;
+    choice = it->second;
+    return true;
+}
+
+void tune_cache_put(int dim, int order, int precision, int mode, int64_t K, int form, TuneChoice choice)
+{
+    std::lock_guard<std::mutex> lk(g_tune_mu);
+    g_tune[TuneKey{dim, order, precision, mode, size_class(K), form}] = choice;
 }
 }  // namespace
 
@@ -212,6 +226,16 @@ struct dgtd_op {
     // from 11.5 MB on they gain 1-10 %).
     bool small_state() const { return (int64_t)real_size() * ndofs < (int64_t)12e6; }
 
+    // Infinity Cache: 256 MB, less a margin (StageArgs::keep_out)
+    bool keep_out() const
+    {
+        return !small_state() && 2 * (int64_t)real_size() * ndofs + record_bytes <= (int64_t)250e6;
+    }
+
+    // The form the stage kernels take by the mesh's size: small element
+    // blocks, plain, shortened first and last stages with or without cached output.
+    int tune_form() const { return small_blocks ? 0 : small_state() ? 1 : keep_out() ? 2 : 3; }
+
     size_t real_size() const { return precision == 64 ? sizeof(double) : sizeof(float); }
     void* state() const { return integrator == DGTD_LSERK4 ? d_buf[cur] : d_buf[0]; }
 
@@ -240,8 +264,7 @@ struct dgtd_op {
         a.small_blocks = small_blocks;
         a.alpha = (T)alpha;
         a.res_in = a.res_out = true;
-        // Infinity Cache: 256 MB, less a margin
-        a.keep_out = !small_state() && 2 * (int64_t)real_size() * ndofs + record_bytes <= (int64_t)250e6;
+        a.keep_out = keep_out();
         a.geo = static_cast<const T*>(d_geo);
         a.conn = d_conn;
         a.mats = static_cast<const T*>(d_mats);
@@ -321,9 +344,8 @@ struct dgtd_op {
     // Times every candidate (the fused LSERK stage for LSERK4 operators -- the
     // launch that steps run; with ca = cb = dt = 0 the state does not change --
     // the operator application otherwise) and keeps the fastest; the state
-    // buffers are zero again afterwards.  The choice is cached per (element
-    // shape, order, precision, stage mode, size class) for the process, so
-    // later operators of the same kind skip the timing.
+    // buffers are zero again afterwards.  The choice is cached for the process
+    // (TuneKey), so later operators of the same kind skip the timing.
     template <typename T>
     void autotune()
     {
@@ -331,7 +353,7 @@ struct dgtd_op {
         const int order = dim == 2 ? T2.p : R.p;
         const int mode_key = integrator == DGTD_LSERK4 ? dgtd::kModeLserk : dgtd::kModeMult;
         TuneChoice cached;
-        if (tune_cache_get(dim, order, precision, mode_key, K, cached)) {
+        if (tune_cache_get(dim, order, precision, mode_key, K, tune_form(), cached)) {
             apply_candidate(cached.best);
             tuning.from_cache = 1;
             tuning.ncandidates = kCandidates;
@@ -399,7 +421,7 @@ struct dgtd_op {
         tuning.ncandidates = kCandidates;
         TuneChoice made{best_c, best_mc, {}};
         for (int c = 0; c < kCandidates; ++c) made.us[c] = tuning.candidate_us[c];
-        tune_cache_put(dim, order, precision, mode_key, K, made);
+        tune_cache_put(dim, order, precision, mode_key, K, tune_form(), made);
     }
 
     // Adds the TF/SF right-hand side at time ts: c_out * S to out and
@@ -1616,7 +1638,7 @@ namespace dgtd {
 bool tuned_mfma_config(int dim, int order, int precision, int64_t K, int* cfg)
 {
     TuneChoice choice;
-    if (!tune_cache_get(dim, order, precision, kModeLserk, K, choice)) {
+    if (!tune_cache_get_any(dim, order, precision, kModeLserk, K, choice)) {
         // a PEC cube of n^3 x 6 tetrahedra (n in 4..32), or a PEC square of
         // n^2 x 2 triangles (n in 8..724)
         std::vector<double> vx;
@@ -1677,10 +1699,11 @@ bool tuned_mfma_config(int dim, int order, int precision, int64_t K, int* cfg)
         o.device = dev;
         dgtd_op* op = nullptr;
         if (dgtd_op_create(&m, &o, &op) != DGTD_OK) return false;
-        const bool got = tune_cache_get(dim, order, precision, kModeLserk, (int64_t)nk, choice);
+        const int form = op->tune_form();
+        const bool got = tune_cache_get(dim, order, precision, kModeLserk, (int64_t)nk, form, choice);
         dgtd_op_destroy(op);
         if (!got) return false;
-        tune_cache_put(dim, order, precision, kModeLserk, K, choice);
+        tune_cache_put(dim, order, precision, kModeLserk, K, form, choice);
     }
     if (choice.best_mfma < 1) return false;
     *cfg = (choice.best_mfma - 1) / 2;

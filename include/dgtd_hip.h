@@ -291,7 +291,8 @@ int dgtd_op_kernel_variant(const dgtd_op* op, int32_t* variant);
  * rounds, three launches then about 1 ms of launches each, the lower mean
  * kept) and the fastest kept; the choice is
  * cached for the process per (element shape, order, precision, stage mode,
- * floor(log2 K)), and later operators of that kind take it without timing.
+ * floor(log2 K), form the kernels take by the mesh's size), and later
+ * operators of that kind take it without timing.
  * Candidates: 0 the per-node stage; 1 + 2c + o the matrix-core stage in
  * configuration c (0: up to 12 FP32 / 8 FP64 waves per block, exterior
  * traces gathered 2 k-steps ahead, residual read at the update; 1: up to 8 /

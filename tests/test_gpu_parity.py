@@ -180,6 +180,22 @@ def test_autotune_picks_a_variant():
     assert g2.tuning()["from_cache"] and g2.kernel_variant() == g.kernel_variant()
 
 
+@pytest.mark.parametrize("below,above", [(1200, 1900), (20000, 30000)])
+def test_autotune_times_each_form(below, above):
+    """Two meshes of one size class (floor(log2 K)), one on either side of a
+    bound where the stage kernels change their form (order 3: element blocks
+    of half the size up to 1,536 tetrahedra, shortened first and last stages
+    from 25,000 in FP32): each is timed, and cached for its own kind."""
+    vx, E, fbc = MG.cube_mesh(18, 1.0, "pec")
+    tuned = []
+    for K in (below, above, below, above):
+        g = D.HesthavenEvolution(vx, E[:K], fbc[:K], 3, precision=32, kernel="auto")
+        tuned.append(g.tuning())
+    assert tuned[2]["from_cache"] and tuned[3]["from_cache"]
+    assert tuned[2]["candidates_us"] == tuned[0]["candidates_us"] != tuned[1]["candidates_us"]
+    assert tuned[3]["candidates_us"] == tuned[1]["candidates_us"]
+
+
 @pytest.mark.parametrize("precision", [32, 64])
 @pytest.mark.parametrize("order", [2, 3, 4, 5])
 def test_every_candidate_same_bits(order, precision):
