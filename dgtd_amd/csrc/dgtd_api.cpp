@@ -342,10 +342,11 @@ struct dgtd_op {
     }
 
     // Times every candidate (the fused LSERK stage for LSERK4 operators -- the
-    // launch that steps run; with ca = cb = dt = 0 the state does not change --
-    // the operator application otherwise) and keeps the fastest; the state
-    // buffers are zero again afterwards.  The choice is cached for the process
-    // (TuneKey), so later operators of the same kind skip the timing.
+    // launch of a step's middle stages; with ca = 1, cb = dt = 0 neither state
+    // nor residual changes -- the operator application otherwise) and keeps the
+    // fastest; the state buffers are zero again afterwards.  The choice is
+    // cached for the process (TuneKey), so later operators of the same kind
+    // skip the timing.
     template <typename T>
     void autotune()
     {
@@ -367,11 +368,11 @@ struct dgtd_op {
         if (integrator == DGTD_LSERK4) {
             mode = dgtd::kModeLserk;
             a.res = static_cast<T*>(d_buf[2]);
-            a.ca = T(0);
+            a.ca = T(1);
             a.cb = T(0);
             a.dt = T(0);
         }
-        // The candidates are timed on noise, not on the zeroed buffers: zeros
+        // State and residual hold noise, not the zeros they start with: zeros
         // toggle no bits, the card clocks higher and the vector stage gains
         // more than the matrix cores do (order 3 FP32, 303,918 tetrahedra: 209
         // against 214 us on zeros, 237 against 206 us on fields).
