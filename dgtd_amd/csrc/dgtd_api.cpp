@@ -812,6 +812,7 @@ void upload_tensor(dgtd_op* op, int p, const std::vector<double>& host_geo, cons
                    const double* sigma, const std::vector<double>& eps, const std::vector<int>& fmask,
                    const std::vector<int>& perm)
 {
+    if (!dgtd::tensor_faces_match(op->dim, p, fmask)) throw std::logic_error("tensor element face table");
     hip_check(hipDeviceGetAttribute(&op->cus, hipDeviceAttributeMultiprocessorCount, op->device), "compute units");
     const int K = op->K, n1 = p + 1, stride = (int)(host_geo.size() / K);
     std::vector<double> geo((size_t)(stride + 1) * K);

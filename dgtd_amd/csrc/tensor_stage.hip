@@ -207,27 +207,22 @@ __global__ __launch_bounds__(kThreads) void tensor_stage(StageArgs<T> a)
             rhs[x] = ieps * (dd(3 + z, y) - dd(3 + y, z)) - sig * uo[x * NE + i];
             rhs[3 + x] = imu * (dd(y, z) - dd(z, y));
         }
-        // lifted fluxes: face f's node on this node's normal line (its
-        // numbering follows the face's vertex cycle), weight M1^-1[line
-        // index][0 or p]
-        auto lift = [&](int f, int line, int end, int b) {
-            const T w = sMi[line * 2 + end];
-            const T* fl = sf + el * 6 * NF + f * NFP + b;
+        // lifted fluxes: face f's node on this node's normal line, weight
+        // M1^-1[line index][0 or p]
+        auto lift = [&](int f) {
+            const int axis = tensor_face_axis(DIM, f);
+            const T w = sMi[(axis == 0 ? ix : axis == 1 ? iy : iz) * 2 + tensor_face_end(DIM, f)];
+            const T* fl = sf + el * 6 * NF + f * NFP + tensor_face_node(DIM, P, f, ix, iy, iz);
 #pragma unroll
             for (int c = 0; c < 6; ++c) rhs[c] += w * fl[c * NF];
         };
+        lift(0);
+        lift(1);
+        lift(2);
+        lift(3);
         if constexpr (DIM == 3) {
-            lift(0, iz, 0, ix + N1 * (P - iy));
-            lift(1, iy, 0, ix + N1 * iz);
-            lift(2, ix, 1, iy + N1 * iz);
-            lift(3, iy, 1, P - ix + N1 * iz);
-            lift(4, ix, 0, P - iy + N1 * iz);
-            lift(5, iz, 1, ix + N1 * iy);
-        } else {
-            lift(0, iy, 0, ix);
-            lift(1, ix, 1, iy);
-            lift(2, iy, 1, P - ix);
-            lift(3, ix, 0, P - iy);
+            lift(4);
+            lift(5);
         }
 #pragma unroll
         for (int c = 0; c < 6; ++c) {

@@ -155,3 +155,19 @@ def test_empty_mesh_is_refused_before_any_device_call():
     rc = _abi.lib().dgtd_op_create(ctypes.byref(desc), ctypes.byref(opts), ctypes.byref(h))
     assert rc == -1 and not h.value
     assert b"at least one element" in _abi.lib().dgtd_last_error()
+
+
+def test_tensor_face_numbering(tmp_path):
+    """The closed forms of the tensor stage's face nodes against the face
+    tables of set-up (tests/cpp/tensor_faces_check.cpp)."""
+    import subprocess
+
+    csrc = os.path.join(ROOT, "dgtd_amd", "csrc")
+    exe = str(tmp_path / "tensor_faces_check")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-pthread", "-I" + os.path.join(ROOT, "include"), "-o", exe,
+                    os.path.join(ROOT, "tests", "cpp", "tensor_faces_check.cpp")]
+                   + [os.path.join(csrc, f) for f in ("hex.cpp", "quad.cpp", "tri.cpp", "mesh.cpp", "reftet.cpp")],
+                   check=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    print(r.stdout, r.stderr)
+    assert r.returncode == 0 and r.stdout == "OK\n"
