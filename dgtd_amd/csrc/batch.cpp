@@ -536,7 +536,7 @@ int batch_error(const std::exception& e)
 
 }  // namespace
 
-// Quadrilaterals and hexahedra run on the assembled (Global) operator only;
+// Quadrilaterals and hexahedra run the Global operator only;
 // the batch advances hesthaven-operator instances.
 constexpr const char* kBatchNoTensorElements =
     "quadrilaterals and hexahedra run the Global operator only (dgtd_op_create: DGTD_KERNEL_CSR, or for hexahedra "
@@ -628,7 +628,7 @@ int dgtd_batch_add_tfsf(dgtd_batch* b, const dgtd_mesh_desc* mesh, const double*
     if (mesh->K < 1 || mesh->nv < 1 || !mesh->vx || !mesh->EToV)
         return dgtd::api_fail(DGTD_E_ARG, "the mesh needs at least one element, its vertices and EToV");
     if (mesh->sigma)
-        return dgtd::api_fail(DGTD_E_UNSUPPORTED, "bulk conductivity needs the assembled operator (DGTD_KERNEL_CSR)");
+        return dgtd::api_fail(DGTD_E_UNSUPPORTED, "bulk conductivity needs the Global operator (DGTD_KERNEL_CSR)");
     if (mesh->order < 1 || mesh->order > dgtd::kMaxBatchOrder)
         return dgtd::api_fail(DGTD_E_UNSUPPORTED, "order must be in 1..5");
     if (!std::isfinite(final_time) || !std::isfinite(dt)) return dgtd::api_fail(DGTD_E_ARG, "bad dt or final_time");

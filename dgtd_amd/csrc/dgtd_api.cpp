@@ -165,8 +165,9 @@ struct dgtd_op {
     int grid_cfg[dgtd::kMfmaConfigs] = {};        // grid per configuration, 0 = does not fit
     // autotuning record: candidates timed at creation (or taken from the cache)
     dgtd_tuning tuning{};
-    // Global operator (DGTD_KERNEL_CSR): matrix-free on tetrahedra and
-    // triangles (sigma/eps_r per element, NULL = no conductivity), else assembled
+    // DGTD_KERNEL_CSR, the Global operator: matrix-free on tetrahedra,
+    // triangles (sigma/eps_r per element in d_sig, NULL = no conductivity) and
+    // quadrilaterals (in their records); assembled on hexahedra
     bool global_free = false;
     void* d_sig = nullptr;
     int64_t* d_rowptr = nullptr;
@@ -650,8 +651,7 @@ dgtd::TriMeshInput tri_input(const dgtd_op* op)
     return in;
 }
 
-// Set-up of a triangle-mesh operator (mesh->dim == 2): reference triangle,
-// geometry and connectivity records, the per-node stage kernel only.
+// Device form of the assembled matrix (kernels.hpp).
 void upload_csr(dgtd_op* op, const dgtd::Csr& A)
 {
     op->nnz = (int64_t)A.val.size();
@@ -688,7 +688,7 @@ int mfma_grid(int64_t K, int waves, int resident)
     return std::max(1, g);
 }
 
-// The stage variant: assembled (CSR), autotuned, or as requested (matrix
+// The stage variant: the Global operator (CSR), autotuned, or as requested (matrix
 // cores in configuration 0 with Morton-ordered tasks).
 template <typename CsrSetup>
 void select_variant(dgtd_op* op, int kernel, CsrSetup csr_setup)
@@ -705,6 +705,8 @@ void select_variant(dgtd_op* op, int kernel, CsrSetup csr_setup)
     }
 }
 
+// Set-up of a triangle-mesh operator (mesh->dim == 2): reference triangle,
+// geometry and connectivity records, per-node and matrix-core stages.
 void create_tri(dgtd_op* op, const dgtd_mesh_desc* mesh, int kernel)
 {
     op->dim = 2;
@@ -716,7 +718,7 @@ void create_tri(dgtd_op* op, const dgtd_mesh_desc* mesh, int kernel)
     op->N = (size_t)op->Np * mesh->K;
     op->ndofs = 6 * (int64_t)op->N;
     // (alpha only guards SMA faces against the centred flux, which the
-    // assembled operator handles: its SMA faces are weighted as at alpha = 1)
+    // Global operator handles: its SMA faces are weighted as at alpha = 1)
     const dgtd::TriMeshData md =
         dgtd::build_tri_mesh(tri_input(mesh), R, kernel == DGTD_KERNEL_CSR ? 1.0 : op->alpha);
     op->max_fscale = md.max_fscale;
@@ -846,7 +848,7 @@ void upload_tensor(dgtd_op* op, int p, const std::vector<double>& host_geo, cons
 void create_quad(dgtd_op* op, const dgtd_mesh_desc* mesh, int kernel)
 {
     if (kernel != DGTD_KERNEL_CSR && kernel != DGTD_KERNEL_AUTO)
-        throw UnsupportedError("quadrilaterals run on the assembled operator (DGTD_KERNEL_CSR)");
+        throw UnsupportedError("quadrilaterals run the Global operator (DGTD_KERNEL_CSR)");
     op->dim = 2;
     op->quad = true;
     op->Q2 = dgtd::build_refquad(mesh->order);
@@ -990,11 +992,10 @@ dgtd::MeshInput mesh_input(const dgtd_mesh_desc* mesh)
     return in;
 }
 
-// Set-up of a hexahedral-mesh operator (dim 3, nvert = 8): the assembled
-// operator only.
-// Hexahedra run the Global operator's flux, either assembled (DGTD_KERNEL_CSR)
-// or matrix-free (DGTD_KERNEL_VALU, which DGTD_KERNEL_AUTO selects:
-// tensor_stage.hip reads no matrix, and the set-up assembles none).
+// Set-up of a hexahedral-mesh operator (dim 3, nvert = 8): the Global
+// operator's flux, either assembled (DGTD_KERNEL_CSR) or matrix-free
+// (DGTD_KERNEL_VALU, which DGTD_KERNEL_AUTO selects: tensor_stage.hip reads no
+// matrix, and the set-up assembles none).
 void create_hex(dgtd_op* op, const dgtd_mesh_desc* mesh, int kernel)
 {
     if (kernel != DGTD_KERNEL_CSR && kernel != DGTD_KERNEL_AUTO && kernel != DGTD_KERNEL_VALU)
@@ -1079,7 +1080,7 @@ int dgtd_op_create(const dgtd_mesh_desc* mesh, const dgtd_opts* opts, dgtd_op** 
         return fail(DGTD_E_ARG, "kernel must be DGTD_KERNEL_AUTO, _VALU, _MFMA or _CSR");
     const bool hexes = mesh->dim != 2 && mesh->nvert == 8;  // their matrix-free stage applies sigma too
     if (mesh->sigma && opts->kernel != DGTD_KERNEL_CSR && !hexes)
-        return fail(DGTD_E_UNSUPPORTED, "bulk conductivity needs the assembled operator (DGTD_KERNEL_CSR)");
+        return fail(DGTD_E_UNSUPPORTED, "bulk conductivity needs the Global operator (DGTD_KERNEL_CSR)");
     if (mesh->dim != 0 && mesh->dim != 2 && mesh->dim != 3) return fail(DGTD_E_ARG, "dim must be 0, 2 or 3");
     if (mesh->nvert != 0 && !(mesh->dim == 2 && (mesh->nvert == 3 || mesh->nvert == 4)) &&
         !(mesh->dim != 2 && (mesh->nvert == 4 || mesh->nvert == 8)))
@@ -1725,7 +1726,7 @@ int dgtd_op_tuning(const dgtd_op* op, dgtd_tuning* out)
 int dgtd_op_set_candidate(dgtd_op* op, int32_t candidate)
 {
     if (!op) return fail(DGTD_E_ARG, "NULL argument");
-    if (op->variant == DGTD_KERNEL_CSR) return fail(DGTD_E_ARG, "assembled operator: no stage candidates");
+    if (op->variant == DGTD_KERNEL_CSR) return fail(DGTD_E_ARG, "Global operator (DGTD_KERNEL_CSR): one stage kernel, no candidates");
     if (op->hex) return fail(DGTD_E_ARG, "hexahedra: one matrix-free stage, no candidates");
     if (candidate < 0 || candidate >= dgtd_op::kCandidates) return fail(DGTD_E_ARG, "candidate out of range");
     int var, cfg;

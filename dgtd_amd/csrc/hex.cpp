@@ -1,6 +1,6 @@
 // Reference hexahedron (tensor product of Gauss-Lobatto-Legendre points,
 // MFEM's L2 Gauss-Lobatto hexahedron: node i + (p+1) j + (p+1)^2 k at
-// (x_i, x_j, x_k), lexicographic) and hexahedral-mesh setup for the assembled
+// (x_i, x_j, x_k), lexicographic) and hexahedral-mesh setup for the Global
 // operator.
 #include "hex.hpp"
 

@@ -1,4 +1,4 @@
-// Hexahedra on the assembled (Global) operator.  The reference's default
+// Hexahedra on the Global operator.  The reference's default
 // evolution operator assembles the DG operator of its L2 Gauss-Lobatto space
 // (EvolutionOptions.h:14, Solver.cpp:27-28) on hexahedral meshes as on
 // tetrahedra; its Solver3DTest cases run it (pec_global_1dot5D and

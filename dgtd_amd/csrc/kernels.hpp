@@ -44,7 +44,7 @@ struct StageArgs {
     const T* mats;       // Dr^T, Ds^T, Dt^T ([j][i] each), then LIFT^T ([m][i])
     const int* tabs;     // Fmask[4*Nfp], then face permutation table [96*Nfp]
     const int* order;    // MFMA variant: processing order of the 16-element tasks (NULL = identity)
-    // assembled (Global) operator, rows and columns in the state layout
+    // assembled Global operator (hexahedra), rows and columns in the state layout
     const int64_t* rowptr;
     const uint16_t* col16;  // element-local column codes (csr_local16)
     const int* etab;        // kCsrTab element ids per 16-DOF block
@@ -66,9 +66,10 @@ struct StageArgs {
     // Per-node stage of tetrahedra: element blocks of half the size (nblk
     // counts those; Shape in stage_body.hpp).
     bool small_blocks;
-    // matrix-free Global operator on tetrahedra and triangles: the kernels'
+    // matrix-free Global operator: on tetrahedra and triangles the kernels'
     // Global variant (SMA faces, codes 3 and 6, upwinded fully whatever alpha;
-    // conductivity) with sigma/eps_r per element in sig (NULL = none)
+    // conductivity) with sigma/eps_r per element in sig (NULL = none); the
+    // tensor-product stage is that operator always, sigma/eps_r in its records
     bool global;
     const T* sig;
 };
@@ -317,7 +318,7 @@ inline int norms_tile(int Np)
 constexpr int kNormsMaxParts = 1024;
 hipError_t norms_scratch(int device, double** ptr);
 
-// Fills p with values in [-1, 1) (the autotuner's test state).
+// Fills p with values in [-1, 1] (the autotuner's test state).
 template <typename T>
 hipError_t launch_fill_noise(T* p, int64_t n, hipStream_t s);
 

@@ -1,6 +1,6 @@
 // Reference quadrilateral (tensor product of Gauss-Lobatto-Legendre points,
 // MFEM's L2 Gauss-Lobatto quadrilateral: node i + (p+1) j at (x_i, x_j),
-// lexicographic) and quadrilateral-mesh setup for the assembled operator.
+// lexicographic) and quadrilateral-mesh setup for the Global operator.
 #include "quad.hpp"
 
 #include <algorithm>

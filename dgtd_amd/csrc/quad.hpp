@@ -1,4 +1,4 @@
-// Quadrilaterals on the assembled (Global) operator.  The reference's default
+// Quadrilaterals on the Global operator.  The reference's default
 // evolution operator assembles the DG operator of its L2 Gauss-Lobatto space
 // (EvolutionOptions.h:14, Solver.cpp:27-28) on quadrilateral meshes as on
 // triangles; its 2D_TFSF_Quads cases run it (ExtensiveCasesTest.cpp:1003,

@@ -146,10 +146,7 @@ template hipError_t launch_norms<float>(const float*, int, int, const double*, c
                                         const double*, const double*, double*, int, double*,
                                         hipStream_t);
 
-// Point probes: one wave per (probe, component) forms
-// sum_n w[probe][n] * q[c*N + elem[probe]*Np + n] in FP64; probes outside
-// the mesh (elem < 0) give NaN.
-// p[i] in [-1, 1), from a mixed counter (the finalising steps of MurmurHash3).
+// p[i] in [-1, 1], from a mixed counter (the finalising steps of MurmurHash3).
 template <typename T>
 __global__ __launch_bounds__(kThreads) void fill_noise(T* p, int64_t n)
 {
@@ -161,6 +158,9 @@ __global__ __launch_bounds__(kThreads) void fill_noise(T* p, int64_t n)
     }
 }
 
+// Point probes: one wave per (probe, component) forms
+// sum_n w[probe][n] * q[c*N + elem[probe]*Np + n] in FP64; probes outside
+// the mesh (elem < 0) give NaN.
 template <typename T>
 __global__ __launch_bounds__(64) void probe_sample(const T* __restrict__ q, size_t N, int Np,
                                                    const int* __restrict__ elem,

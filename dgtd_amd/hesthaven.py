@@ -286,7 +286,7 @@ def mesh_geometry(vx, EToV, face_bc, order, alpha=1.0, eps=None, mu=None):
 
 
 def global_assemble(vx, EToV, face_bc, order, alpha=1.0, eps=None, mu=None, sigma=None, quads=None):
-    """The assembled operator of the "csr" kernel on the host, FP64:
+    """The operator of the "csr" kernel assembled on the host, FP64:
     (rowptr, col, val) of the ndofs x ndofs CSR matrix (the Global operator's
     matrix, DGOperatorFactory::buildGlobalOperator, DGOperatorFactory.h:1428-1600)."""
     m = _Mesh(vx, EToV, face_bc, order, eps, mu, sigma, quads=quads)

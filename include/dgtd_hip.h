@@ -318,7 +318,7 @@ int dgtd_op_tuning(const dgtd_op* op, dgtd_tuning* out);
  * the reference): the candidate numbered as above (0 .. ncandidates-1).
  * DGTD_E_ARG when it does not fit this operator (no matrix-core variant at
  * this order and precision, element order without a Morton permutation) or
- * the operator is assembled (DGTD_KERNEL_CSR).  The matrix-core candidates
+ * the operator is the Global one (DGTD_KERNEL_CSR).  The matrix-core candidates
  * compute the same arithmetic in the same order, so they store identical
  * results; the per-node candidate sums in another order and agrees to
  * rounding (FP64 to 1e-12 of the oracle).  Callers pin one for reproducible
@@ -367,7 +367,7 @@ int dgtd_project_initial_fields(const dgtd_mesh_desc* mesh, const dgtd_initial_f
 
 /* ------------------------------------------------------------------------
  * Case files: the reference's JSON launcher input (driver.cpp:531-706,
- * 940-1035, 1242-1300) as far as the hesthaven and assembled operators run
+ * 940-1035, 1242-1300) as far as the hesthaven and Global operators run
  * it.
  *   solver_options: upwind_alpha, time_step (0 = the reference's automatic rule,
  *                   dgtd_case_time_step), final_time,

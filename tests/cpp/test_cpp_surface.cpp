@@ -1,9 +1,9 @@
 // The C++ TimeDependentOperator surface (include/dgtd_hip.hpp) against the
 // CPU oracle: Mult and an RK4 Solver::run on a 2^3 PEC cavity at p=3, FP64;
-// the assembled (CSR) variant against the oracle's Mult and, with a uniform
+// the Global operator (CSR) against the oracle's Mult and, with a uniform
 // conductivity sigma (eps = 1), against A x - sigma x_E (the conductive term
 // is -sigma/eps on the E DOFs); on a triangle mesh the per-node, matrix-core
-// and assembled variants against each other.  Exit status 0 and "OK".
+// and Global variants against each other.  Exit status 0 and "OK".
 #include <cmath>
 #include <cstdio>
 #include <random>
@@ -68,7 +68,7 @@ int main()
     } catch (const dgtd::Error& e) {
         ok = ok && e.code == DGTD_E_UNSUPPORTED;
     }
-    {  // assembled operator, same mesh
+    {  // Global operator, same mesh
         dgtd::Options oc = opts;
         oc.kernel = DGTD_KERNEL_CSR;
         dgtd::HesthavenEvolutionHip csr(mesh, oc);

@@ -290,7 +290,7 @@ def read_gmsh22_2d(path):
     return np.array(xyz), np.array(tris, dtype=np.int64), segs
 
 
-# ---- quadrilaterals (parallelograms, the assembled operator) ----
+# ---- quadrilaterals (parallelograms, the Global operator) ----
 
 QUAD_EDGES = ((0, 1), (1, 2), (2, 3), (3, 0))
 

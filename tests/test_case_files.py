@@ -698,7 +698,7 @@ def test_hexahedral_tfsf_case(tmp_path):
 
 
 def test_case_kernel_choice_counts_interior_sma(tmp_path):
-    """kernel "auto" takes the assembled operator where the Global operator's
+    """kernel "auto" takes the Global operator ("csr") where its
     SMA weighting differs from the matrix-free one: SMA faces at alpha != 1,
     interior SMA (code 6) as well as boundary SMA, as the launcher decides."""
     shutil.copy(os.path.join(CASES, "2D_TFSF_IntBoundary.msh"), tmp_path / "2D_TFSF_IntBoundary.msh")

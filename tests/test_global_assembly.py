@@ -1,4 +1,4 @@
-"""The assembled operator of the "csr" kernel (the Global operator's matrix,
+"""The operator of the "csr" kernel, assembled (the Global operator's matrix,
 DGOperatorFactory::buildGlobalOperator, DGOperatorFactory.h:1428-1600),
 checked on the host.
 

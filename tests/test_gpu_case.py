@@ -312,7 +312,7 @@ def test_2d_tfsf_quads_like_reference(tmp_path, alpha, dt):
     """ExtensiveCasesTest 2D_TFSF_Centered_Quads (alpha 0, time step 5e-3) and
     2D_TFSF_Upwind_Quads (the case as written: alpha 1, time step 0.01)
     (test/cases/ExtensiveCasesTest.cpp:1003-1157): quadrilaterals on the
-    Global (assembled) operator; the Gaussian plane wave enters through the
+    Global operator; the Gaussian plane wave enters through the
     TF/SF line x = 1 and bounces in the PEC/PMC guide; tolerance 1e-2."""
     opts = dict(upwind_alpha=alpha)
     if dt is not None:
@@ -329,7 +329,7 @@ def test_2d_tfsf_quads_like_reference(tmp_path, alpha, dt):
 
 
 def test_launcher_runs_quad_case(tmp_path):
-    """The C++ launcher takes the quadrilateral case to the assembled
+    """The C++ launcher takes the quadrilateral case to the Global
     operator and matches the library run."""
     out = tmp_path / "exp"
     r = subprocess.run([LAUNCH, QUADS2D, "--final-time", "0.5", "--out", str(out)], capture_output=True, text=True,
@@ -349,7 +349,7 @@ def test_launcher_runs_hexahedral_case(tmp_path):
     Gmsh mesh of 10 x 2 x 2 hexahedra on [0,1] x [0,0.4] x [0,0.4] with
     MakeCartesian3D's side tags (PEC z, PMC y, SMA x), the Gaussian E_z pulse,
     order 3, time step 7e-3, final time 1, point probes at x = 0 and x = 1.
-    The launcher runs it on the assembled operator; its PointProbe files show
+    The launcher runs it on the Global operator; its PointProbe files show
     the two halves leaving through the SMA ends (E_z = 0.5, H_y = +-0.5 at the
     sample nearest t = 0.5; zero at t = 1; tolerance 1e-2), and its final norm
     matches the library run."""

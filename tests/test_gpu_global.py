@@ -1,6 +1,6 @@
-"""The assembled ("csr") operator on the GPU, through the C ABI: the
-reference's Global path (GlobalEvolution::Mult, GlobalEvolution.cpp:628-1088)
-as one fused CSR SpMV + stage-update kernel.
+"""The Global operator (kernel "csr") on the GPU, through the C ABI: the
+reference's Global path (GlobalEvolution::Mult, GlobalEvolution.cpp:628-1088),
+on tetrahedra and triangles without the matrix.
 
 Bars: FP64 Mult equals the oracle's Mult (no conductivity; SMA faces as the
 Global operator weights them, see tests/test_global_assembly.py) and the host CSR

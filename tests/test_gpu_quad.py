@@ -1,4 +1,4 @@
-"""Quadrilaterals on the GPU: the assembled operator (DGTD_KERNEL_CSR), the
+"""Quadrilaterals on the GPU: the Global operator (DGTD_KERNEL_CSR), the
 operator the reference runs on quadrilateral meshes (its Global operator,
 GlobalEvolution::Mult, GlobalEvolution.cpp:628-1088).
 
@@ -59,7 +59,7 @@ def test_quad_mult_matches_oracle(order):
 
 def test_quad_kernel_choice_and_node_positions():
     vx, E, bc = MG.quad_mesh(3, 2, bc="pec", stretch=0.2, shear=0.2)
-    op = D.HesthavenEvolution(vx, E, bc, 3, quads=True)  # kernel "auto" takes the assembled operator
+    op = D.HesthavenEvolution(vx, E, bc, 3, quads=True)  # kernel "auto" takes the Global operator
     assert op.kernel_variant() == "csr"
     ref = O2.Operator2D(vx, E, bc, 3, quads=True)
     pos = op.node_positions()
@@ -67,7 +67,7 @@ def test_quad_kernel_choice_and_node_positions():
     np.testing.assert_allclose(pos[1], ref.pos[..., 1], atol=1e-14)
     assert op.max_fscale() == pytest.approx(ref.max_fscale(), rel=1e-14)
     for kernel in ("valu", "mfma"):
-        with pytest.raises(D.DgtdError, match="assembled operator") as ei:
+        with pytest.raises(D.DgtdError, match="Global operator") as ei:
             D.HesthavenEvolution(vx, E, bc, 3, kernel=kernel, quads=True)
         assert ei.value.code == -4
 
