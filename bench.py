@@ -9,11 +9,11 @@ components), dt from the Hesthaven rule dt = 1/(max fscale * p^2).
 
 The headline value is FP32 DOF*RK-stages/s; the FP64 path runs the same steps
 beside it and the relative L2 difference FP32 vs FP64 is reported.  roofline
-takes the algorithmic bytes per element per stage (24*Np*s + 27*s + 32) and
+takes the algorithmic bytes per element per stage (21.6*Np*s + 27*s + 32) and
 flops (36 Np^2 + 48 Np Nfp + 240 Nfp + 96 Np) times K over the average
 stage-kernel duration from HIP events on the operator's stream, and reports
 the resource whose ideal time is the longer (at order 4 in FP32 the matrix
-cores: 95 us against 86 us of HBM traffic) with the HBM figures beside it.  cpu_baseline times the CPU FP64 oracle (a restatement of the
+cores: 95 us against 78 us of HBM traffic) with the HBM figures beside it.  cpu_baseline times the CPU FP64 oracle (a restatement of the
 reference algorithm) with OpenMP on the host cores for one LSERK4 step of the
 same mesh.
 """
@@ -127,12 +127,13 @@ def mass_norm(D, vx, E, fbc, order, v):
 
 def work_per_element(order, precision):
     """Algorithmic bytes and flops per tetrahedron per stage (the library's
-    dgtd_op_work_per_element formula): 24 Np s + 27 s + 32 bytes and
+    dgtd_op_work_per_element formula): 21.6 Np s + 27 s + 32 bytes (24 Np s in
+    the batch's order-1 stage, which moves the residual in every stage) and
     36 Np^2 + 48 Np Nfp + 240 Nfp + 96 Np flops."""
     s = 4 if precision == 32 else 8
     Np = (order + 1) * (order + 2) * (order + 3) // 6
     Nfp = (order + 1) * (order + 2) // 2
-    return 24 * Np * s + 27 * s + 32, 36 * Np * Np + 48 * Np * Nfp + 240 * Nfp + 96 * Np
+    return (24 if order == 1 else 21.6) * Np * s + 27 * s + 32, 36 * Np * Np + 48 * Np * Nfp + 240 * Nfp + 96 * Np
 
 
 def stage_kernel(op, order, precision, dim=3):
@@ -275,15 +276,17 @@ def bench_c3(D, args):
 
 
 def bench_global(D, args, shape="tet"):
-    """The assembled (Global) operator with conductivity: PEC cavity [0,1]^3,
+    """The Global operator (kernel "csr") with conductivity: PEC cavity [0,1]^3,
     12^3 hexes x 6 = 10,368 tets, p=3, eps_r ~ U[1,4], a conducting slab
     (sigma = 2 for x < 1/2), Ez Gaussian pulse, 100 LSERK4 steps in FP32 and
-    FP64 through the fused CSR SpMV stage kernel.  shape "quad": the same on
-    a PEC/PMC square [0,1]^2 of 256^2 quadrilaterals; "hex": on a PEC cavity
-    [0,1]^3 of 32^3 hexahedra (the reference runs its quadrilateral and
-    hexahedral meshes on this operator), p=3; --size overrides the cells per
-    edge.  CPU leg: the same FP64 CSR product on one host core (scipy), the
-    Global operator's SparseMatrix::Mult."""
+    FP64 through the per-node stage's Global form, without the matrix.  shape
+    "quad": the same on a PEC/PMC square [0,1]^2 of 256^2 quadrilaterals
+    through the tensor-product stage; "hex": on a PEC cavity [0,1]^3 of 32^3
+    hexahedra through the fused CSR SpMV stage and, beside it, the
+    tensor-product stage (the reference runs its quadrilateral and hexahedral
+    meshes on this operator), p=3; --size overrides the cells per edge.  CPU
+    leg: the FP64 product with the assembled matrix on one host core (scipy),
+    the Global operator's SparseMatrix::Mult."""
     order = 3
     steps = args.steps
     rng = np.random.default_rng(args.seed)
@@ -313,7 +316,7 @@ def bench_global(D, args, shape="tet"):
     x0 = D.project_initial_fields(vx, E, order, src)
     dof = 6 * np_ * K
     out = {"workload": f"{mesh}, p={order}, eps_r~U[1,4], "
-                       f"sigma=2 for x<1/2, Ez Gaussian, {steps} LSERK4 steps, assembled CSR operator", "dof": dof}
+                       f"sigma=2 for x<1/2, Ez Gaussian, {steps} LSERK4 steps, Global operator", "dof": dof}
     states = {}
 
     def timed(op, prec, name):
@@ -331,14 +334,15 @@ def bench_global(D, args, shape="tet"):
         state = op.get_state()
         op.close()
         return state, {"value": dof * 5 * steps / wall, "unit": "DOF*RK-stages/s", "wall_s": wall,
-                       "kernel_avg_us": us, "kernel": f"{name}<{'float' if prec == 32 else 'double'},LSERK>",
+                       "kernel_avg_us": us, "kernel": f"{name}<{'float' if prec == 32 else 'double'},LSERK{',GLOBAL' if shape == 'tet' else ''}>",
                        "algorithmic_bytes_per_launch": b * K,
                        "hbm_frac": b * K / (us * 1e-6) / 1e9 / HBM_PEAK_GBS,
                        "energy_initial": e0, "energy_final": nm["energy"], "nonfinite": nm["nonfinite"]}
 
     for prec in (32, 64):
         op = D.GlobalEvolution(vx, E, fbc, order, eps=eps, sigma=sigma, precision=prec, integrator="lserk4")
-        states[prec], out[f"fp{prec}"] = timed(op, prec, "csr_stage")
+        states[prec], out[f"fp{prec}"] = timed(op, prec, {"quad": "tensor_stage", "hex": "csr_stage"}.get(
+            shape, "dg_stage_kernel"))
     if shape == "hex":  # the matrix-free hexahedron stage on the same operator
         for prec in (32, 64):
             op = D.HesthavenEvolution(vx, E, fbc, order, eps=eps, sigma=sigma, precision=prec,
@@ -495,7 +499,7 @@ def main():
                     choices=["c1", "c2", "c3", "c4", "c5", "tri", "global", "quad", "hex"],
                     help="c2 (default, the headline): 32^3 cavity p=4; c3: 48^3 SMA box with random eps, "
                          "p=3, 2000 steps; c4: 64 uneven cavities batched; c5: Poisson serving stream; "
-                         "tri: the 2D operator on 524,288 triangles, p=4; global: the assembled CSR operator "
+                         "tri: the 2D operator on 524,288 triangles, p=4; global: the Global operator "
                          "on 10,368 tets with conductivity; quad: the same on 256^2 quadrilaterals; hex: on "
                          "32^3 hexahedra")
     ap.add_argument("--size", type=int, default=0, help="global/quad/hex: cells per edge (0 = the workload's own)")

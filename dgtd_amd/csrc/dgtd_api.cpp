@@ -227,6 +227,13 @@ struct dgtd_op {
     // from 11.5 MB on they gain 1-10 %).
     bool small_state() const { return (int64_t)real_size() * ndofs < (int64_t)12e6; }
 
+    // Whether LSERK4's first stage reads no residual and its last leaves none
+    // (the assembled stage keeps both: run-time tests cost it more).
+    bool short_stages() const
+    {
+        return integrator == DGTD_LSERK4 && !small_state() && (variant != DGTD_KERNEL_CSR || global_free);
+    }
+
     // Infinity Cache: 256 MB, less a margin (StageArgs::keep_out)
     bool keep_out() const
     {
@@ -470,8 +477,8 @@ struct dgtd_op {
                 a.ca = (T)kA[s];
                 a.cb = (T)kB[s];
                 a.unstable = s == 4 ? d_unstable : nullptr;  // the step's new state
-                a.res_in = s != 0 || small_state();
-                a.res_out = s != 4 || small_state();
+                a.res_in = s != 0 || !short_stages();
+                a.res_out = s != 4 || !short_stages();
                 launch<T>(a, dgtd::kModeLserk);
                 // res' = res + dt S, q' = q + b res'  =>  q' += b dt S
                 tfsf<T>(t + kC[s] * dt, a.out, kB[s] * dt, a.res_out ? a.res : nullptr, dt, stream);
@@ -1765,24 +1772,29 @@ int dgtd_op_work_per_element(const dgtd_op* op, double* bytes, double* flops)
         if (flops) *flops = 2.0 * nnz_e + 4.0 * rows;
         return DGTD_OK;
     }
+    // values of a state buffer a step moves per stage: four passes over the six
+    // components (state, residual in and out, output; classic RK4's four stages
+    // come to the same), 18 instead of 20 in five stages without the first
+    // residual read and the last store
+    const double vecs = op->short_stages() ? 21.6 : 24.0;
     if (op->hex) {  // matrix-free hexahedra: state vectors, 36-value record, 12 connectivity ints
         const double n1 = op->H3.p + 1.0;
-        if (bytes) *bytes = 24.0 * Np * s + 36.0 * s + 48.0;
+        if (bytes) *bytes = vecs * Np * s + 36.0 * s + 48.0;
         if (flops) *flops = Np * (36.0 * n1 + 198.0) + 240.0 * Nfp;
         return DGTD_OK;
     }
     if (op->quad) {  // matrix-free quadrilaterals: state vectors, 19-value record, 8 connectivity ints
         const double n1 = op->Q2.p + 1.0;
-        if (bytes) *bytes = 24.0 * Np * s + 19.0 * s + 32.0;
+        if (bytes) *bytes = vecs * Np * s + 19.0 * s + 32.0;
         if (flops) *flops = Np * (24.0 * n1 + 150.0) + 160.0 * Nfp;
         return DGTD_OK;
     }
     if (op->dim == 2) {  // triangles: 2 derivative directions, 3 edges, 15-value record
-        if (bytes) *bytes = 24.0 * Np * s + 15.0 * s + 24.0;
+        if (bytes) *bytes = vecs * Np * s + 15.0 * s + 24.0;
         if (flops) *flops = 24.0 * Np * Np + 36.0 * Np * Nfp + 150.0 * Nfp + 96.0 * Np;
         return DGTD_OK;
     }
-    if (bytes) *bytes = 24.0 * Np * s + 27.0 * s + 32.0;
+    if (bytes) *bytes = vecs * Np * s + 27.0 * s + 32.0;
     if (flops) *flops = 36.0 * Np * Np + 48.0 * Np * Nfp + 240.0 * Nfp + 96.0 * Np;
     return DGTD_OK;
 }

@@ -325,7 +325,9 @@ int dgtd_op_tuning(const dgtd_op* op, dgtd_tuning* out);
  * timing or bits. */
 int dgtd_op_set_candidate(dgtd_op* op, int32_t candidate);
 
-/* Algorithmic HBM bytes and flops per element per stage for this operator. */
+/* Algorithmic HBM bytes and flops per element per stage for this operator (the
+ * mean over a step's stages: above 12 MB per state buffer LSERK4 reads no
+ * residual in its first stage and stores none in its last). */
 int dgtd_op_work_per_element(const dgtd_op* op, double* bytes, double* flops);
 
 /* Structured cube generator: n^3 hexahedra on [0,L]^3, each split into six

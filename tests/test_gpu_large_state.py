@@ -155,3 +155,18 @@ def test_steps_past_the_infinity_cache(shape, kernel):
     x = np.random.default_rng(2).standard_normal(op.ndofs)
     dt = 0.2 * np.linalg.norm(x) / np.linalg.norm(op.mult(x))
     check_steps(op, 64, "lserk4", x, 0.0, dt)
+
+
+@pytest.mark.parametrize("shape,kernel", CASES)
+def test_bytes_per_stage(shape, kernel):
+    """A step of five stages moves 18 passes over the six components above 12
+    MB per state buffer and 20 below it (always 20 with the assembled matrix;
+    RK4: 16 in four stages)."""
+    records = {"tet": 27 * 8 + 32, "triangle": 15 * 8 + 24, "quad": 19 * 8 + 32, "hex": 36 * 8 + 48}[shape]
+    for megabytes, integrator, passes in ((12, "lserk4", 18 / 5), (0.1, "lserk4", 4), (12, "rk4", 4)):
+        op = operator(shape, kernel, 64, mesh(shape, megabytes, 64), integrator)
+        b = op.work_per_element()[0]
+        if (shape, kernel) == ("hex", "csr"):
+            assert b > 4 * 6 * NODES[shape] * 8
+        else:
+            assert b == pytest.approx(passes * 6 * NODES[shape] * 8 + records, rel=1e-14)
