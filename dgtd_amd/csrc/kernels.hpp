@@ -55,7 +55,8 @@ struct StageArgs {
     // LSERK: whether the stage reads and leaves the residual.  The first stage
     // of a step has ca = 0 and the next step starts afresh, so a step needs no
     // residual read in its first stage and none stored by its last: 18
-    // passes over a state buffer per step instead of 20.
+    // passes over a state buffer per step instead of 20.  (The assembled stage
+    // always reads and stores it.)
     bool res_in, res_out;
     // Whether the stage output is stored for reuse (else it streams past the
     // caches): while the state, the output and the element records fit the 256
